@@ -45,6 +45,7 @@ UNITS = [
     ("vx3h_server.cpp", "cxx", []),
     ("vx3h_tune.cpp", "cxx", []),
     ("vx3h_tile.cpp", "cxx", []),
+    ("vx3h_steptile.cpp", "cxx", []),
 ]
 
 

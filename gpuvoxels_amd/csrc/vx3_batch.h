@@ -81,7 +81,8 @@ template <typename T> struct DevBatch {
     int vHi, lHi, nSims;      // high-water marks: kernels cover [0, vHi) / [0, lHi) / [0, nSims)
     int solo;                 // >= 0: only this simulation takes the step (on the per-step kernels,
                               // whichever path it was admitted to); -1: every stream-path simulation;
-                              // -2: every simulation, resident ones included
+                              // -2: every simulation, resident ones included; -3: every
+                              // stream-path simulation, those of the fused kernel too
 };
 
 // Tables of a tiled resident launch (one workgroup per tile, TileDesc); unused by
@@ -100,6 +101,23 @@ struct TileArgs {
     int repair;              // 1: run only the simulations whose last launch diverged (divergence word
                              // = 1 + the launch step), up to that step's link pass
     int flag0;               // index in sync of workgroup 0's arrival flag
+};
+
+// Tile records of the fused per-step kernel (vx3_tilestep.inl).  The state has two copies: a
+// step reads the one and writes the other.
+struct TsArgs {
+    const TsTile* tiles;      // per workgroup
+    char* stat;               // [record] TsStat::BYTES
+    char* state;              // [record][2] TsState::BYTES
+    TsAux* aux;               // [record]
+    const double* ph;         // distinct actuation phases per simulation
+    const int* o2p;           // per simulation, place of each voxel
+    const int* tab;           // per simulation, its voxel and link material constants (the LDS tables' image)
+    TsCtl* ctl;               // [2][ctlCap]
+    TsReport* report;         // [2][ctlCap]
+    int ctlCap;
+    int par;                  // parity of the step within its call: which copies it reads
+    unsigned seq0;            // load: the number its report carries
 };
 
 }  // namespace vx3

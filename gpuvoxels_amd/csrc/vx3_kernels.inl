@@ -27,7 +27,8 @@ __device__ __forceinline__ bool simRunning(const DevBatch<real>& b, int s) {
     const int f = b.sims[s].flags;
     if (b.solo >= 0) return s == b.solo && !(f & SC_COL_GROW);
     if (b.solo == -2) return !(f & SC_COL_GROW);   // every simulation, resident ones included
-    return !(f & (SC_RESIDENT | SC_COL_GROW));
+    if (b.solo == -3) return !(f & (SC_RESIDENT | SC_COL_GROW));   // those of the fused kernel too
+    return !(f & (SC_RESIDENT | SC_TILESTEP | SC_COL_GROW));
 }
 
 // Precision-dependent transcendentals.  The FP64 state path rounds like the host C
@@ -1444,6 +1445,25 @@ __device__ void blockCloseness(const DevBatch<real>& b, const SimCtl& sc, double
     __syncthreads();
 }
 
+// A center-of-mass sample: the history of three and the angle between the last two
+// displacements (VX3_VoxelyzeKernel.cu:314-334).
+// (SimCtl, or the fused kernel's TsCtl.)
+template <typename Ctl> __device__ __forceinline__ void comSampled(Ctl& sc, const double com[3]) {
+    sc.angleSamples++;
+    for (int k = 0; k < 3; k++) { sc.comH0[k] = sc.comH1[k]; sc.comH1[k] = sc.com[k]; sc.com[k] = com[k]; }
+    const double* A = sc.comH0; const double* B = sc.comH1; const double* C = sc.com;
+    const bool bc = B[0] == C[0] && B[1] == C[1] && B[2] == C[2];
+    const bool ab = A[0] == B[0] && A[1] == B[1] && A[2] == B[2];
+    if (bc || ab || sc.angleSamples < 3) sc.recentAngle = 0;
+    else {
+        double d1[3] = {B[0] - A[0], B[1] - A[1], B[2] - A[2]}, d2[3] = {C[0] - B[0], C[1] - B[1], C[2] - B[2]};
+        double dot = d1[0] * d2[0] + d1[1] * d2[1] + d1[2] * d2[2];
+        double l1 = sqrt((A[0] - B[0]) * (A[0] - B[0]) + (A[1] - B[1]) * (A[1] - B[1]) + (A[2] - B[2]) * (A[2] - B[2]));
+        double l2 = sqrt((B[0] - C[0]) * (B[0] - C[0]) + (B[1] - C[1]) * (B[1] - C[1]) + (B[2] - C[2]) * (B[2] - C[2]));
+        sc.recentAngle = acos(dot / (l1 * l2));
+    }
+}
+
 // Per-simulation bookkeeping after the voxel pass (doTimeStep tail, VX3_VoxelyzeKernel.cu:241,279,314-334,352,
 // and the stop test the driver loop makes before the next step, VX3_SimulationManager.cu:62-64).
 __global__ void __launch_bounds__(256) k_control(DevBatch<real> b) {
@@ -1486,19 +1506,7 @@ __global__ void __launch_bounds__(256) k_control(DevBatch<real> b) {
         return;
     }
     if (sample) {
-        sc.angleSamples++;
-        for (int k = 0; k < 3; k++) { sc.comH0[k] = sc.comH1[k]; sc.comH1[k] = sc.com[k]; sc.com[k] = com[k]; }
-        const double* A = sc.comH0; const double* B = sc.comH1; const double* C = sc.com;
-        const bool bc = B[0] == C[0] && B[1] == C[1] && B[2] == C[2];
-        const bool ab = A[0] == B[0] && A[1] == B[1] && A[2] == B[2];
-        if (bc || ab || sc.angleSamples < 3) sc.recentAngle = 0;
-        else {
-            double d1[3] = {B[0] - A[0], B[1] - A[1], B[2] - A[2]}, d2[3] = {C[0] - B[0], C[1] - B[1], C[2] - B[2]};
-            double dot = d1[0] * d2[0] + d1[1] * d2[1] + d1[2] * d2[2];
-            double l1 = sqrt((A[0] - B[0]) * (A[0] - B[0]) + (A[1] - B[1]) * (A[1] - B[1]) + (A[2] - B[2]) * (A[2] - B[2]));
-            double l2 = sqrt((B[0] - C[0]) * (B[0] - C[0]) + (B[1] - C[1]) * (B[1] - C[1]) + (B[2] - C[2]) * (B[2] - C[2]));
-            sc.recentAngle = acos(dot / (l1 * l2));
-        }
+        comSampled(sc, com);
         if (sc.closeR > 0) { sc.closeness = closeness; sc.closePairs = closePairs; }
     }
     if (reinit) {   // InitializeCenterOfMass: the last sampled center of mass

@@ -3,6 +3,7 @@
 #define VX_NS k_f32
 #include "vx3_kernels.inl"
 #include "vx3_resident.inl"
+#include "vx3_tilestep.inl"
 #include "vx3_launch.h"
 
 #include "vx3_stream_launch.inl"

@@ -45,6 +45,12 @@ hipError_t launchTiled(const DevBatch<double>& b, hipStream_t s, int shape, cons
                        int nSteps, hipEvent_t* ev = nullptr);
 hipError_t tiledOccupancy(const DevBatch<float>& b, int shape, int* perCU);
 hipError_t tiledOccupancy(const DevBatch<double>& b, int shape, int* perCU);
+// The fused per-step kernel over the tiles ts.tiles[0, nTiles): batch arrays into the tile
+// records (TS_LOAD), one step (TS_STEP), and back (TS_STORE).  shape: 0 for tiles of at most
+// VX3_TS_OWN slots (owned and halo), 1 for tiles of at most VX3_TS_CUT owned voxels, 2 any.
+enum { TS_LOAD, TS_STEP, TS_STORE };
+hipError_t launchTileStep(const DevBatch<float>& b, const TsArgs& ts, hipStream_t s, int what, int nTiles, int shape);
+hipError_t launchTileStep(const DevBatch<double>& b, const TsArgs& ts, hipStream_t s, int what, int nTiles, int shape);
 void launchDt(const DevBatch<float>& b, hipStream_t s, int s0, int s1);
 void launchDt(const DevBatch<double>& b, hipStream_t s, int s0, int s1);
 // copies the link end loads of voxels [0, nv) from src (slot stride srcFs) to dst (slot

@@ -58,6 +58,27 @@ void launchCopyLoads(const DevBatch<VX_REAL>& b, hipStream_t s, const void* src,
                            (VX_REAL*)dst, dstFs, nv);
 }
 
+// LDS strides of the fused kernel's shapes: slots, owned voxels
+#define VX3_TS_SHAPES(F) F(0, VX3_TS_OWN, VX3_TS_OWN) F(1, VX3_TS_SLOTS, VX3_TS_CUT) F(2, VX3_TS_SLOTS, VX3_TS_OWN)
+
+hipError_t launchTileStep(const DevBatch<VX_REAL>& b, const TsArgs& ts, hipStream_t s, int what, int nTiles, int shape) {
+    if (nTiles <= 0) return hipSuccess;
+    if (what == TS_LOAD) hipLaunchKernelGGL(VX_NS::k_ts_load, dim3(nTiles), dim3(VX3_TS_BLOCK), 0, s, b, ts);
+    else if (what == TS_STORE) hipLaunchKernelGGL(VX_NS::k_ts_store, dim3(nTiles), dim3(VX3_TS_BLOCK), 0, s, b, ts);
+#define VX3_TS_CASE(I, S, N)                                                                                       \
+    else if (shape == I) {                                                                                         \
+        auto kern = VX_NS::k_ts_step<S, N>;                                                                        \
+        const size_t lds = VX_NS::TsShape<S, N>::bytes;                                                            \
+        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+        if (e != hipSuccess) return e;                                                                             \
+        hipLaunchKernelGGL(kern, dim3(nTiles), dim3(VX3_TS_BLOCK), lds, s, b, ts);                                 \
+    }
+    VX3_TS_SHAPES(VX3_TS_CASE)
+#undef VX3_TS_CASE
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 void launchDt(const DevBatch<VX_REAL>& b, hipStream_t s, int s0, int s1) {
     if (s1 > s0) hipLaunchKernelGGL(VX_NS::k_dt, dim3(s1 - s0), dim3(256), 0, s, b, s0, s1);
 }

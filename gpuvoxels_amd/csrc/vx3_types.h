@@ -54,7 +54,11 @@ enum { SC_VARY = 1, SC_EXPANSION = 2, SC_DIVERGED_PENDING = 4, SC_POISSON = 8, S
        SC_NEARDIRTY = 1 << 19,  // this step regenerates the nearby lists from the current links
        SC_LINKS_DONE = 1 << 20,    // stood still for a collision table after this step's link pass:
                                    // the step resumes after the link pass (its end loads are kept)
-       SC_NEARMASK = 1 << 21 };    // nearby sets also held as lattice-offset bit masks (nearMask)
+       SC_NEARMASK = 1 << 21,      // nearby sets also held as lattice-offset bit masks (nearMask)
+       SC_TILESTEP = 1 << 22,      // steps on the fused per-step kernel (k_ts_step) in calls of several steps
+       SC_TSLOADED = 1 << 23,      // TsCtl only: its state is in the fused kernel's tile arrays,
+       SC_TSPARV = 1 << 24,        // which of the two copies of its voxel state is current,
+       SC_TSPARL = 1 << 25 };      // and of its link state
 #define VX3_COL_HBLOCK 1024     // hash buckets per scan block; a simulation's buckets are whole blocks
 
 // A voxel's nearby set (the surface voxels within the link-hop radius) as a bit mask over
@@ -105,6 +109,9 @@ struct LinkMatDev {                 // CVX_MaterialLink derived constants (VX_Ma
     float strainData[VX3_MAX_CURVE];
     float stressData[VX3_MAX_CURVE];
 };
+
+// the fused per-step kernel's LDS tables: up to 8 voxel and 16 link material constants
+#define VX3_TS_TAB (8 * sizeof(VoxMatDev) + 16 * sizeof(LinkMatDev))
 
 struct ExtDev {                     // CVX_External (VX_External.h:34-94)
     int dofFixed;
@@ -169,6 +176,77 @@ struct SimCtl {                     // one running simulation (VX3_VoxelyzeKerne
     int nlMax, safety;
     int atOff[5], atLen[5];
     int scanDone;                    // bucket blocks of the current rebuild scanned so far (k_col_bscan)
+};
+
+// What changes of a simulation's control state from step to step on the fused per-step
+// kernel.  Two copies per simulation: a step reads the one, as of the step before's start,
+// applies what that step's tiles reported, and leaves the result in the other.  A report is
+// the step's number in the word for its kind, so no word is ever cleared.
+struct TsCtl {
+    double t, recentAngle;
+    double com[3], comH0[3], comH1[3];
+    int state, steps, flags, angleSamples, rebuilds;
+    unsigned seq;                    // number of the next step to report
+    float prevDt;
+    int sampled;                     // the step before summed the center of mass
+};
+struct TsReport { unsigned diverged, stale, grow; int nbUsed; };   // nbUsed: list entries handed out by that step's rebuild
+
+// One tile of a simulation on the fused per-step kernel (vx3h_steptile.h): a workgroup of
+// VX3_TS_BLOCK threads steps the nOwn voxels it owns.
+#define VX3_TS_BLOCK 256             // threads
+#define VX3_TS_OWN 288               // owned voxels at most: a body of up to this many stays whole,
+                                     // its voxels past the threads' number taking a second round
+#define VX3_TS_CUT 192               // voxels of a block cut from a larger body: the last wave
+                                     // computes the links that come in across its faces
+#define VX3_TS_SLOTS 448             // owned + halo voxels at most, of which halo VX3_TS_OWN
+struct TsTile {
+    int sim;                         // simulation slot
+    int tile, nTiles;                // index in its simulation, tiles of its simulation
+    int rec;                         // its record in the tile pool (those of a simulation are consecutive)
+    int nOwn, nSurf, nHalo, nIn[3];  // owned voxels, the first nSurf on the surface; halo; incoming links per axis
+    int ctl;                         // its simulation's index in ctl, report and tab
+    int ph0, nPh;                    // its distinct actuation phases ph[ph0 .. ph0 + nPh)
+    int o0;                          // its o2p range: place of each sim-local voxel
+    int pad[2];
+};
+// A place is a record and a slot of it: record << VX3_TS_SLOT_BITS | slot.
+#define VX3_TS_SLOT_BITS 9
+
+// A tile record: rows of VX3_TS_OWN elements, one per owned slot.  TsStat (byte offsets) is
+// written at admission up to ST_END; the rest and TsState belong to a call.
+struct TsStat {
+    static constexpr int R4 = 4 * VX3_TS_OWN;
+    static constexpr int ST = 0;               // voxel material | phase << 4 | external << 10 | link material of axis a << (12 + 4a)
+    static constexpr int NBR = R4;             // 3 rows of unsigned short: tile slot at the link's positive end, 0xFFFF = no link
+    static constexpr int ORIG = NBR + 6 * VX3_TS_OWN;   // voxel (batch index), -1 = none
+    static constexpr int HALO = ORIG + R4;     // place of each halo voxel
+    static constexpr int IN = HALO + R4;       // 3 rows' room: incoming links, axis by axis: halo tile slot | owned slot << 16
+    static constexpr int LINK = IN + 3 * R4;   // 3 rows: link (batch index), -1 = none
+    static constexpr int IJK = LINK + 3 * R4;  // row of pairs of words: lattice index from the simulation's lowest, x | y << 16
+                                               // and z | (121 x + 11 y + z) << 16 (modulo 2^16; see NearBitTable's index)
+    static constexpr int ST_END = IJK + 2 * R4;
+    static constexpr int LS = ST_END;          // 3 rows: strain of the last step
+    static constexpr int LW = LS + 3 * R4;     // 3 rows: position at the last list rebuild
+    static constexpr int NBC = LW + 3 * R4, NBS = NBC + R4;   // partner list: entries, start in nbList
+    static constexpr int BYTES = (NBS + R4 + 255) / 256 * 256;
+};
+template <int REAL> struct TsState {   // one of the two copies; REAL = bytes of the state precision
+    static constexpr int RR = REAL * VX3_TS_OWN, R4 = 4 * VX3_TS_OWN;
+    static constexpr int VR = 0;               // 13 rows: position, orientation, linear, angular momentum
+    static constexpr int LR = 13 * RR;         // per axis 9 rows: previous pos2, angle2v, angle1v (large-angle links only)
+    static constexpr int VF = LR + 27 * RR;    // 4 rows: thermal factor, Poisson strain
+    static constexpr int LF = VF + 4 * R4;     // per axis 2 rows: maxStrain, strainOffset (the latter: non-linear materials only)
+    static constexpr int VI = LF + 6 * R4;     // voxel flags
+    static constexpr int LB = VI + R4;         // 3 rows of bytes: LF_* bits
+    static constexpr int BYTES = (LB + 3 * VX3_TS_OWN + 255) / 256 * 256;
+};
+struct TsAux {                       // per tile, by parity of the step that writes it
+    // at its last list rebuild: bounds of its surface voxels (lowest x, y, z, [3], highest) and
+    // of each 64 of them (lowest, highest); [3]: how far one of them has moved since
+    float hull[2][8];
+    float box[2][VX3_TS_BLOCK / 64][6];
+    double part[2][4];               // centre-of-mass partial sums
 };
 
 // One tile of a simulation that the resident kernel runs on several workgroups (tiled

@@ -24,6 +24,7 @@
 #include "vx3_launch.h"
 #include "vx3h_build.h"
 #include "vx3h_internal.h"
+#include "vx3h_steptile.h"
 #include "vx3h_tile.h"
 
 namespace vx3 {
@@ -114,6 +115,9 @@ struct SlotHost {
     int tv0 = 0, tvN = 0, tl0 = 0, tlN = 0, tx0 = 0, txN = 0, tp0 = 0;   // its ranges in the tile pools
     bool oneTile = false;        // a one-workgroup simulation with one-tile tables in the pools
     int axisLinks = 0;           // links on its busiest axis
+    std::vector<TsTile> stepTiles;   // steps on the fused per-step kernel as these tiles
+    int maxStepSlots = 0, maxStepOwn = 0;
+    int ts0 = 0, tq0 = 0, tqN = 0, to0 = 0, tc0 = 0;   // its ranges in that kernel's pools
     std::vector<int> ijk;
     std::vector<int> matid;
     std::vector<int> measured;   // per voxel
@@ -217,6 +221,22 @@ struct vx3h_batch {
     hipStream_t tileStream = nullptr;
     hipEvent_t tileJoin = nullptr;
     bool tilePending = false;
+    // fused per-step kernel: simulations too large for the resident kernels, in calls of
+    // at least VX3_TS_MIN_STEPS steps
+    std::vector<int> stepSims;                   // slots, in admission order
+    bool stepDirty = false;
+    TsTile* dStepTiles = nullptr; size_t capStepTiles = 0;
+    int nStepTiles = 0;
+    int stepShape = 0;
+    TsArgs ts{};
+    DevPool stepTilePool, stepPhasePool, stepO2pPool, stepCtlPool;
+    int stepCtlCap = 0;                          // control states allocated
+    int stepPar = 0;                             // parity of the next step of the call
+    unsigned stepSeq = 1;                        // report numbers used so far
+    hipGraphExec_t stepGraphExec = nullptr;
+    hipGraph_t stepGraph = nullptr;
+    int stepGraphSteps = 0;
+    long stepGraphLayout = -1;
     // while tiled simulations run, the one-workgroup simulations without collisions run in
     // the same cooperative launches as one-tile entries (a cooperative launch can only
     // start once every CU it needs is free: beside them it would wait for theirs)
@@ -231,7 +251,7 @@ struct vx3h_batch {
     // graph of `graphSteps` steps, valid for one layout version
     hipGraphExec_t graphExec = nullptr;
     hipGraph_t graph = nullptr;
-    int graphSteps = 0;
+    int graphSteps = 0, graphSolo = -1;
     long layout = 0, graphLayout = -1;
     // launch timing (vx3h_batch_set_timing)
     bool timing = false;
@@ -294,6 +314,15 @@ void initSpecs(vx3h_batch* b) {
     b->tileXchPool.arrs = {{(void**)&b->dXch, 2 * VX3_XCH_STRIDE * R}};   // one record, both parities
     b->tilePartPool.arrs = {{(void**)&b->dPart, 8 * sizeof(double)}};    // one tile, both parities
     b->tileXchPool.minCap = b->tilePartPool.minCap = 256;
+    TsArgs& t = b->ts;
+    b->stepTilePool.arrs = {{(void**)&t.stat, TsStat::BYTES}, {(void**)&t.state, 2 * (R == 8 ? TsState<8>::BYTES : TsState<4>::BYTES)},
+                            {(void**)&t.aux, sizeof(TsAux)}};
+    b->stepPhasePool.arrs = {{(void**)&t.ph, 8}};
+    b->stepO2pPool.arrs = {{(void**)&t.o2p, 4}};
+    b->stepCtlPool.arrs = {{(void**)&t.tab, VX3_TS_TAB}};
+    b->stepTilePool.minCap = 32;
+    b->stepPhasePool.minCap = 64;
+    b->stepCtlPool.minCap = 16;
     L(&d.lneg, 4, 1, false); L(&d.lpos, 4, 1, false); L(&d.lmeta, 4, 1, false); L(&d.lsim, 4, 1, false); L(&d.lflags, 4, 1, false);
     L(&d.q2x, R, 1, false); L(&d.q2y, R, 1, false); L(&d.q2z, R, 1, false);
     L(&d.a1x, R, 1, false); L(&d.a1y, R, 1, false); L(&d.a1z, R, 1, false);
@@ -477,22 +506,25 @@ vx3h_status uploadNearMasks(vx3h_batch* b, int v0, int nv, const int* ijk, const
 StepOpts stepOpts(const vx3h_batch* b);
 vx3h_status placeLoads(vx3h_batch* b, bool scratch);
 
-vx3h_status launchSteps(vx3h_batch* b, int n) {
+// n steps of the per-step kernels; solo as DevBatch::solo
+vx3h_status launchSteps(vx3h_batch* b, int n, int solo) {
     const StepOpts o = stepOpts(b);
+    DevBatch<float> v = b->db;
+    v.solo = solo;
     for (int i = 0; i < n; i++) {
-        if (b->realSize == 4) launchStep(b->db, b->stream, o);
-        else launchStep(*reinterpret_cast<DevBatch<double>*>(&b->db), b->stream, o);
+        if (b->realSize == 4) launchStep(v, b->stream, o);
+        else launchStep(*reinterpret_cast<DevBatch<double>*>(&v), b->stream, o);
     }
     HIPCHK(hipGetLastError());
     return VX3H_OK;
 }
 
-vx3h_status ensureGraph(vx3h_batch* b, int steps) {
-    if (b->graphExec && b->graphLayout == b->layout && b->graphSteps == steps) return VX3H_OK;
+vx3h_status ensureGraph(vx3h_batch* b, int steps, int solo) {
+    if (b->graphExec && b->graphLayout == b->layout && b->graphSteps == steps && b->graphSolo == solo) return VX3H_OK;
     if (b->graphExec) { HIPCHK(hipGraphExecDestroy(b->graphExec)); b->graphExec = nullptr; }
     if (b->graph) { HIPCHK(hipGraphDestroy(b->graph)); b->graph = nullptr; }
     HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    vx3h_status st = launchSteps(b, steps);
+    vx3h_status st = launchSteps(b, steps, solo);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (st != VX3H_OK) return st;
@@ -501,6 +533,7 @@ vx3h_status ensureGraph(vx3h_batch* b, int steps) {
     HIPCHK(hipGraphInstantiate(&b->graphExec, g, nullptr, nullptr, 0));
     b->graphLayout = b->layout;
     b->graphSteps = steps;
+    b->graphSolo = solo;
     return VX3H_OK;
 }
 
@@ -625,6 +658,193 @@ vx3h_status syncTiles(vx3h_batch* b) {
     if (!T.empty()) HIPCHK(hipMemcpy(b->dTiles, T.data(), T.size() * sizeof(TileDesc), hipMemcpyHostToDevice));
     b->tileDirty = false;
     return VX3H_OK;
+}
+
+// ---- the fused per-step kernel (vx3_tilestep.inl)
+
+// the control states and reports for the control pool's capacity (contents not kept: a call
+// sets them up)
+vx3h_status stepCtl(vx3h_batch* b) {
+    TsArgs& t = b->ts;
+    if (b->stepCtlCap == b->stepCtlPool.cap) return VX3H_OK;
+    const size_t c = b->stepCtlPool.cap;
+    HIPCHK(hipStreamSynchronize(b->stream));
+    b->stepCtlCap = 0;
+    if (t.ctl) { HIPCHK(hipFree(t.ctl)); t.ctl = nullptr; }
+    if (t.report) { HIPCHK(hipFree(t.report)); t.report = nullptr; }
+    HIPCHK(hipMalloc((void**)&t.ctl, c * 2 * sizeof(TsCtl)));
+    HIPCHK(hipMalloc((void**)&t.report, c * 2 * sizeof(TsReport)));
+    HIPCHK(hipMemsetAsync(t.report, 0, c * 2 * sizeof(TsReport), b->stream));   // report numbers start at 1
+    b->stepCtlCap = t.ctlCap = (int)c;
+    b->layout++;
+    return VX3H_OK;
+}
+
+// device memory a plan's growth of the pools needs (old and new arrays exist side by side
+// while one is replaced)
+size_t stepGrowth(const vx3h_batch* b, const StepTilePlan& p, int nv) {
+    size_t tot = 0;
+    auto grow = [&](const DevPool& q, size_t n) {
+        if ((size_t)q.ra.hi + n <= (size_t)q.cap) return;
+        const size_t c = std::max((size_t)q.ra.hi + n, (size_t)std::max(2 * q.cap, q.minCap));
+        for (const auto& a : q.arrs) tot += c * a.second;
+    };
+    grow(b->stepTilePool, p.tiles.size());
+    grow(b->stepPhasePool, RES_MAX_PHASES);
+    grow(b->stepO2pPool, nv);
+    grow(b->stepCtlPool, 1);
+    return tot;
+}
+
+void releaseStep(vx3h_batch* b, SlotHost& sh) {
+    b->stepTilePool.ra.release(sh.ts0, (int)sh.stepTiles.size());
+    b->stepPhasePool.ra.release(sh.tq0, sh.tqN);
+    b->stepO2pPool.ra.release(sh.to0, sh.nv);
+    b->stepCtlPool.ra.release(sh.tc0, 1);
+    sh.stepTiles.clear();
+}
+
+// A simulation's step tiles: ranges in the pools, tables uploaded.  sh.v0, l0 and nv are set.
+vx3h_status placeStep(vx3h_batch* b, SlotHost& sh, const HostModel& H, StepTilePlan& p) {
+    const int T = (int)p.tiles.size();
+    std::vector<double> phases;
+    std::vector<int> phaseOf(H.nv), o2p(H.nv);
+    {
+        std::map<uint64_t, int> seen;   // distinct phase offsets, as bit patterns
+        uint64_t last = 0;
+        int lastAt = -1;
+        for (int v = 0; v < H.nv; v++) {
+            uint64_t u;
+            memcpy(&u, &H.phase[v], 8);
+            if (lastAt < 0 || u != last) {
+                auto it = seen.find(u);
+                if (it == seen.end()) { it = seen.emplace(u, (int)phases.size()).first; phases.push_back(H.phase[v]); }
+                last = u;
+                lastAt = it->second;
+            }
+            phaseOf[v] = lastAt;
+        }
+    }
+    sh.tqN = (int)phases.size();
+    vx3h_status e;
+    if ((e = poolAlloc(b, b->stepTilePool, T, sh.ts0)) || (e = poolAlloc(b, b->stepPhasePool, sh.tqN, sh.tq0)) ||
+        (e = poolAlloc(b, b->stepO2pPool, H.nv, sh.to0)) || (e = poolAlloc(b, b->stepCtlPool, 1, sh.tc0)) || (e = stepCtl(b)))
+        return e;
+    if (b->stepTilePool.ra.hi > (INT32_MAX >> VX3_TS_SLOT_BITS)) FAILV(VX3H_ENOMEM, "too many step tiles");
+    std::vector<char> tab(VX3_TS_TAB, 0);   // by the simulation's own material indices
+    memcpy(tab.data(), H.vmats.data(), H.vmats.size() * sizeof(VoxMatDev));
+    memcpy(tab.data() + RES_MAX_VMATS * sizeof(VoxMatDev), H.lmats.data(), H.lmats.size() * sizeof(LinkMatDev));
+    for (int t = 0; t < T; t++) {
+        unsigned* st = p.row<unsigned>(t, TsStat::ST);
+        int *orig = p.row<int>(t, TsStat::ORIG), *link = p.row<int>(t, TsStat::LINK), *halo = p.row<int>(t, TsStat::HALO);
+        for (int i = 0; i < p.tiles[t].nOwn; i++) {
+            const int v = orig[i];
+            unsigned w = (unsigned)H.vmat[v] | ((unsigned)phaseOf[v] << 4) | (H.vext[v] >= 0 ? 1u << 10 : 0u);
+            for (int a = 0; a < 3; a++) {
+                int& l = link[a * VX3_TS_OWN + i];
+                if (l < 0) continue;
+                w |= (unsigned)H.lmat[l] << (12 + 4 * a);
+                l += sh.l0;
+            }
+            st[i] = w;
+            o2p[v] = (sh.ts0 + t) << VX3_TS_SLOT_BITS | i;
+            orig[i] += sh.v0;
+        }
+        for (int h = 0; h < p.tiles[t].nHalo; h++) halo[h] += sh.ts0 << VX3_TS_SLOT_BITS;
+    }
+    const TsArgs& t = b->ts;
+    char* stage;   // the records' first part, one strided copy
+    if ((e = stageAlloc(b, p.stat.size(), &stage))) return e;
+    memcpy(stage, p.stat.data(), p.stat.size());
+    HIPCHK(hipMemcpy2DAsync(t.stat + (size_t)sh.ts0 * TsStat::BYTES, TsStat::BYTES, stage, TsStat::ST_END, TsStat::ST_END, T,
+                            hipMemcpyHostToDevice, b->stream));
+    if ((e = upload(b, (char*)t.tab + (size_t)sh.tc0 * VX3_TS_TAB, tab.data(), tab.size())) ||
+        (e = upload(b, (void*)(t.ph + sh.tq0), phases.data(), phases.size() * 8)) || (e = upload(b, (void*)(t.o2p + sh.to0), o2p.data(), o2p.size() * 4)))
+        return e;
+    sh.stepTiles = p.tiles;
+    sh.maxStepSlots = p.maxSlots;
+    sh.maxStepOwn = p.maxOwn;
+    return VX3H_OK;
+}
+
+// The launch's tile list, after a simulation joined or left.
+vx3h_status syncStep(vx3h_batch* b) {
+    if (!b->stepDirty) return VX3H_OK;
+    std::vector<TsTile> T;
+    int slots = 1, own = 1;
+    for (int s : b->stepSims) {
+        const SlotHost& sh = b->slots[s];
+        for (TsTile d : sh.stepTiles) {
+            d.sim = s;
+            d.rec = sh.ts0 + d.tile;
+            d.ctl = sh.tc0;
+            d.ph0 = sh.tq0;
+            d.nPh = sh.tqN;
+            d.o0 = sh.to0;
+            T.push_back(d);
+        }
+        slots = std::max(slots, sh.maxStepSlots);
+        own = std::max(own, sh.maxStepOwn);
+    }
+    HIPCHK(hipStreamSynchronize(b->stream));
+    vx3h_status st = growDev(&b->dStepTiles, &b->capStepTiles, T.size());
+    if (st) return st;
+    if (!T.empty()) HIPCHK(hipMemcpy(b->dStepTiles, T.data(), T.size() * sizeof(TsTile), hipMemcpyHostToDevice));
+    b->nStepTiles = (int)T.size();
+    b->ts.tiles = b->dStepTiles;
+    b->stepShape = slots <= VX3_TS_OWN ? 0 : own <= VX3_TS_CUT ? 1 : 2;   // smallest LDS, so most workgroups per CU
+    b->stepDirty = false;
+    b->layout++;
+    return VX3H_OK;
+}
+
+// n launches of the fused kernel (what: TS_LOAD and TS_STORE once, around a call's steps)
+vx3h_status launchStepTiles(vx3h_batch* b, int what, int n) {
+    TsArgs a = b->ts;
+    if (what == TS_LOAD) {
+        b->stepPar = 0;
+        a.seq0 = b->stepSeq;
+        b->stepSeq++;
+    }
+    for (int i = 0; i < n; i++) {
+        a.par = b->stepPar;
+        const hipError_t e = b->realSize == 4
+            ? launchTileStep(b->db, a, b->stream, what, b->nStepTiles, b->stepShape)
+            : launchTileStep(*reinterpret_cast<DevBatch<double>*>(&b->db), a, b->stream, what, b->nStepTiles, b->stepShape);
+        if (e != hipSuccess) FAILV(VX3H_EDEVICE, std::string("step-tile launch failed: ") + hipGetErrorString(e));
+        if (what == TS_STEP) b->stepPar ^= 1;
+    }
+    return VX3H_OK;
+}
+
+// n steps of the fused kernel, in graphs of up to 32 (an even number, from parity 0)
+vx3h_status runStepTiles(vx3h_batch* b, int n) {
+    b->stepSeq += (unsigned)n;
+    if (!b->cfg.use_graph) return launchStepTiles(b, TS_STEP, n);
+    vx3h_status st;
+    if (n > 0 && b->stepPar) {
+        if ((st = launchStepTiles(b, TS_STEP, 1))) return st;
+        n--;
+    }
+    const int G = std::min(n & ~1, 32);
+    if (G > 0 && !(b->stepGraphExec && b->stepGraphLayout == b->layout && (b->stepGraphSteps == G || b->stepGraphSteps == 32))) {
+        if (b->stepGraphExec) { HIPCHK(hipGraphExecDestroy(b->stepGraphExec)); b->stepGraphExec = nullptr; }
+        if (b->stepGraph) { HIPCHK(hipGraphDestroy(b->stepGraph)); b->stepGraph = nullptr; }
+        HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+        st = launchStepTiles(b, TS_STEP, G);
+        hipGraph_t g = nullptr;
+        const hipError_t e = hipStreamEndCapture(b->stream, &g);
+        if (st) return st;
+        if (e != hipSuccess) FAILV(VX3H_EDEVICE, std::string("graph capture failed: ") + hipGetErrorString(e));
+        b->stepGraph = g;
+        HIPCHK(hipGraphInstantiate(&b->stepGraphExec, g, nullptr, nullptr, 0));
+        b->stepGraphLayout = b->layout;
+        b->stepGraphSteps = G;
+    }
+    if (G > 0)
+        for (; n >= b->stepGraphSteps; n -= b->stepGraphSteps)
+            if (hipGraphLaunch(b->stepGraphExec, b->stream) != hipSuccess) FAILV(VX3H_EDEVICE, "graph launch failed");
+    return launchStepTiles(b, TS_STEP, n);
 }
 
 vx3h_status takeEvent(vx3h_batch* b, hipEvent_t& e) {
@@ -805,7 +1025,9 @@ extern "C" vx3h_status vx3h_batch_destroy(vx3h_batch* b) {
     }
     if (b->tileStream) { hipStreamSynchronize(b->tileStream); hipStreamDestroy(b->tileStream); }
     if (b->tileJoin) hipEventDestroy(b->tileJoin);
-    for (void* p : {(void*)b->dTiles, (void*)b->dSync}) if (p) hipFree(p);
+    for (void* p : {(void*)b->dTiles, (void*)b->dSync, (void*)b->dStepTiles, (void*)b->ts.ctl, (void*)b->ts.report}) if (p) hipFree(p);
+    if (b->stepGraphExec) hipGraphExecDestroy(b->stepGraphExec);
+    if (b->stepGraph) hipGraphDestroy(b->stepGraph);
     if (b->forkEv) hipEventDestroy(b->forkEv);
     if (b->graphExec) hipGraphExecDestroy(b->graphExec);
     if (b->graph) hipGraphDestroy(b->graph);
@@ -815,7 +1037,8 @@ extern "C" vx3h_status vx3h_batch_destroy(vx3h_batch* b) {
     for (int* p : b->dResLists) if (p) hipFree(p);
     if (b->db.colAny) hipFree(b->db.colAny);
     for (DevPool* pl : {&b->nbPool, &b->hashPool, &b->nearPool, &b->cellPool, &b->tgtPool, &b->attPool, &b->pairPool,
-                        &b->tileSlotPool, &b->tileLinkPool, &b->tileXchPool, &b->tilePartPool})
+                        &b->tileSlotPool, &b->tileLinkPool, &b->tileXchPool, &b->tilePartPool, &b->stepTilePool, &b->stepPhasePool,
+                        &b->stepO2pPool, &b->stepCtlPool})
         for (auto& a : pl->arrs) if (*a.first) hipFree(*a.first);
     for (auto& pr : b->evUsed) { b->evPool.push_back(pr.first); b->evPool.push_back(pr.second); }
     for (hipEvent_t e : b->evPool) hipEventDestroy(e);
@@ -843,7 +1066,15 @@ struct PreparedSim {
     int vmax = 0, lax = 0, cap = 0;
     TilePlan plan;
     bool planOk = false;
+    bool stepPlanned = false;      // the plan below is the fused per-step kernel's
+    StepTilePlan stepPlan;
 };
+
+bool stepPlanOf(const HostModel& H, StepTilePlan* out) {
+    std::vector<char> interior(H.nv);
+    for (int v = 0; v < H.nv; v++) interior[v] = (H.vflags[v] & VF_INTERIOR) != 0;
+    return planStepTiles(H.nv, H.ijk.data(), H.nl, H.lneg.data(), H.lpos.data(), H.voxelLinks.data(), interior.data(), out);
+}
 
 // the tile plan a simulation of this model gets if it is too large for one workgroup
 // (planned for any model over the tiled shape's one-workgroup capacity without collisions;
@@ -867,6 +1098,15 @@ vx3h_status prepareSim(const vx3h_batch* b, const vx3h_sim_desc* desc, PreparedS
             p->planOk = planTiles(H.nv, H.ijk.data(), H.nl, H.lneg.data(), H.lpos.data(), H.laxis.data(), vmax, lax,
                                   b->tileCap, &p->plan);
         }
+    }
+    // too large for the resident kernels: the step tiles, where admission may use them
+    if (H.nv > 0 && b->tiledShape >= 0 && !(p->planned && p->planOk && p->plan.tiles.size() > 1)) {
+        const ResidentShapeInfo& r = b->shapes[b->tiledShape];
+        int perAxis[3] = {0, 0, 0};
+        for (int i = 0; i < H.nl; i++) perAxis[H.laxis[i]]++;
+        const int lax = r.block * r.lpa;
+        if (H.nv > r.block * r.vpt || perAxis[0] > lax || perAxis[1] > lax || perAxis[2] > lax)
+            p->stepPlanned = stepPlanOf(H, &p->stepPlan);
     }
     *out = p;
     return VX3H_OK;
@@ -1120,6 +1360,22 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
         b->cfg.path == VX3H_PATH_RESIDENT)
         FAILV(VX3H_EUNSUPPORTED,
               "detach, attach, secondary experiments, signals, target contacts and close pairs run on the stream path");
+    // too large for the resident kernels, without topology changes or extra forces: the
+    // fused per-step kernel, where the device memory that later admissions may still claim
+    // (the rest of the budget) leaves room for its tile arrays
+    StepTilePlan splan;
+    bool stepped = shape < 0 && !tiles && NV > 0 && resOk && b->cfg.path != VX3H_PATH_RESIDENT;
+    if (stepped) {
+        if (pre && pre->stepPlanned) splan = std::move(pre->stepPlan);
+        else stepped = stepPlanOf(H, &splan);
+    }
+    if (stepped) {
+        size_t freeB = 0, totB = 0;
+        HIPCHK(hipMemGetInfo(&freeB, &totB));
+        const size_t later = b->budget > b->bytesUsed + need ? b->budget - b->bytesUsed - need : 0;
+        const size_t grow = stepGrowth(b, splan, NV);
+        if (grow > 0 && freeB < later + grow) stepped = false;
+    }
     // control block
     SimCtl c;
     memset(&c, 0, sizeof(c));
@@ -1134,7 +1390,7 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     c.tInit = H.tInit;
     c.state = VX3H_SIM_RUNNING;
     c.maxSteps = H.maxSteps;
-    c.flags = H.flags | (shape >= 0 || tiles ? SC_RESIDENT : 0);
+    c.flags = H.flags | (shape >= 0 || tiles ? SC_RESIDENT : 0) | (stepped ? SC_TILESTEP : 0);
     c.v0 = v0; c.nv = NV; c.l0 = l0; c.nl = NL;
     c.stopOff = tok0;
     c.mat0 = mat0;
@@ -1358,6 +1614,10 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
         b->resLists[sh.shape].push_back(s);
         b->resDirty = true;
         b->tileDirty = true;
+    } else if (stepped) {
+        if (vx3h_status st = placeStep(b, sh, H, splan)) return st;
+        b->stepSims.push_back(s);
+        b->stepDirty = true;
     }
     else b->nStreamSims++;
     sh.vlinks = H.voxelLinks;
@@ -1394,6 +1654,16 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
 #undef FILL
 }  // namespace vx3
 
+// Shortest call in steps that the fused per-step kernel takes: copying the state into the tile
+// arrays and back costs about as much as what it saves in three to four steps.  Measured on
+// MI355X, us per call, per-step kernels -> fused:
+//   steps                               4             5             6             8
+//   64x64x32, FP64, collisions    272 -> 253    337 -> 290    406 -> 327    532 -> 400
+//   64x64x1, FP32                 131 -> 137    160 -> 160    189 -> 180    248 -> 225
+//   2,048 balls of 257, FP64      962 -> 996            - (a list rebuild)
+//   300 balls of 123, FP32        141 -> 135            -     446 -> 199    513 -> 240
+#define VX3_TS_MIN_STEPS 6
+
 extern "C" vx3h_status vx3h_batch_step(vx3h_batch* b, int n_steps) {
     if (!b || n_steps < 0) FAILV(VX3H_EINVAL, "bad argument");
     HIPCHK(hipSetDevice(b->device));
@@ -1407,26 +1677,47 @@ extern "C" vx3h_status vx3h_batch_step(vx3h_batch* b, int n_steps) {
     }
     const int chunk = b->cfg.steps_per_launch > 0 ? b->cfg.steps_per_launch : 1000;
     if (vx3h_status ps = placeLoads(b, false)) return ps;
+    // The fused kernel takes its simulations in calls of enough steps to pay for copying the
+    // state into the tile arrays and back; shorter calls leave them to the per-step kernels,
+    // and so does the first step of a simulation that stood still after its link pass.
+    const bool resume = b->resumePending;
     b->resumePending = false;   // every waiting simulation resumes in the first step below
-    for (int done = 0; done < n_steps;) {
-        const int c = std::min(chunk, n_steps - done);
-        vx3h_status st = launchResidentAll(b, c, nullptr);
-        if (!st && b->nStreamSims > 0) {
+    const bool fused = !b->stepSims.empty() && n_steps >= VX3_TS_MIN_STEPS;
+    if (fused)
+        if (vx3h_status st = syncStep(b)) return st;
+    bool loaded = false;
+    vx3h_status st = VX3H_OK;
+    for (int done = 0; done < n_steps && !st;) {
+        const bool plain = !b->stepSims.empty() && (!fused || (resume && done == 0));
+        const int c = fused && plain ? 1 : std::min(chunk, n_steps - done);
+        st = launchResidentAll(b, c, nullptr);
+        if (!st && (b->nStreamSims > 0 || plain)) {
+            const int solo = plain ? -3 : -1;
             if (b->cfg.use_graph) {
                 const int G = std::min(c, 32);
-                st = ensureGraph(b, G);
+                st = ensureGraph(b, G, solo);
                 for (int r = 0; !st && r < c / G; r++)
                     if (hipGraphLaunch(b->graphExec, b->stream) != hipSuccess) { g_err = "graph launch failed"; st = VX3H_EDEVICE; }
-                if (!st && c % G) st = launchSteps(b, c % G);
-            } else st = launchSteps(b, c);
+                if (!st && c % G) st = launchSteps(b, c % G, solo);
+            } else st = launchSteps(b, c, solo);
+        }
+        if (!st && fused && !plain) {
+            if (!loaded) {
+                st = launchStepTiles(b, TS_LOAD, 1);
+                loaded = true;
+            }
+            if (!st) st = runStepTiles(b, c);
         }
         // the main stream waits for the resident launches, also after a failure
         const vx3h_status js = joinResident(b);
-        if (st) return st;
-        if (js) return js;
+        if (!st) st = js;
         done += c;
     }
-    return VX3H_OK;
+    if (loaded) {
+        const vx3h_status ls = launchStepTiles(b, TS_STORE, 1);
+        if (!st) st = ls;
+    }
+    return st;
 }
 
 namespace {
@@ -1649,6 +1940,25 @@ extern "C" vx3h_status vx3h_batch_kernel_times(vx3h_batch* b, int n_steps, doubl
         avg_ms[5] += ms;
     }
     for (auto& e : rev) hipEventDestroy(e);
+    if (!b->stepSims.empty()) {   // the fused per-step kernel: the steps' summed duration
+        if ((st = syncStep(b))) return st;
+        hipEvent_t e0, e1;
+        HIPCHK(hipEventCreate(&e0));
+        HIPCHK(hipEventCreate(&e1));
+        if ((st = launchStepTiles(b, TS_LOAD, 1))) return st;
+        HIPCHK(hipEventRecord(e0, b->stream));
+        b->stepSeq += (unsigned)n_steps;
+        st = launchStepTiles(b, TS_STEP, n_steps);
+        HIPCHK(hipEventRecord(e1, b->stream));
+        const vx3h_status ls = launchStepTiles(b, TS_STORE, 1);
+        if (st || (st = ls)) return st;
+        HIPCHK(hipEventSynchronize(e1));
+        float ms = 0;
+        HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+        avg_ms[5] += ms;
+        hipEventDestroy(e0);
+        hipEventDestroy(e1);
+    }
     return VX3H_OK;
 }
 
@@ -1989,6 +2299,10 @@ extern "C" vx3h_status vx3h_sim_retire(vx3h_batch* b, int slot) {
         L.erase(std::remove(L.begin(), L.end(), slot), L.end());
         b->resDirty = true;
         b->tileDirty = true;
+    } else if (!sh.stepTiles.empty()) {
+        b->stepSims.erase(std::remove(b->stepSims.begin(), b->stepSims.end(), slot), b->stepSims.end());
+        releaseStep(b, sh);
+        b->stepDirty = true;
     } else b->nStreamSims--;
     if (sh.oneTile) {
         b->tileSlotPool.ra.release(sh.tv0, sh.tvN);

@@ -1,0 +1,31 @@
+// vx3h_steptile.h -- cutting a simulation into tiles for the fused per-step kernel.
+#ifndef VX3H_STEPTILE_H
+#define VX3H_STEPTILE_H
+#include <cstddef>
+#include <vector>
+#include "vx3_types.h"
+
+namespace vx3 {
+
+// The tiles of one simulation, one workgroup of VX3_TS_BLOCK threads each.  A tile owns up
+// to VX3_TS_BLOCK voxels, one per thread, or a whole body of up to VX3_TS_OWN (at most
+// VX3_TS_BLOCK of them on the surface); its slots are the owned voxels (surface voxels first,
+// each group body by body and ascending) and then the halo: the other ends of their links.  stat holds per tile
+// the rows of TsStat up to ST_END, with voxels, links and tiles counted within the simulation
+// (row ST is the caller's to fill); each link belongs to the slot of its negative end.
+struct StepTilePlan {
+    std::vector<TsTile> tiles;   // tile, nTiles, nOwn, nSurf, nHalo, nIn; the rest is the caller's to fill
+    std::vector<char> stat;
+    int maxSlots = 0, maxOwn = 0;
+    template <typename E> E* row(int tile, int off) { return (E*)(stat.data() + (size_t)tile * TsStat::ST_END + off); }
+};
+
+// Cuts the voxels [0, nv) (lattice indices ijk; vlinks: six link indices per voxel, -1 =
+// none; interior per voxel) joined by links into tiles: connected bodies that fit a tile
+// stay whole, near ones together where they are many and small; larger ones are cut into compact lattice blocks.  False
+// for an empty simulation or a lattice of more than 2^16 along an axis.
+bool planStepTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos, const int* vlinks,
+                   const char* interior, StepTilePlan* out);
+
+}  // namespace vx3
+#endif

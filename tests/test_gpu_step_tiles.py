@@ -1,0 +1,148 @@
+"""The fused per-step kernel (one launch per step, a workgroup per tile) against the
+per-step kernels, which vx3h_batch_step_noalloc runs on every simulation: the same
+operations in the same order, so the same bits -- positions, orientations, momenta, flags,
+thermal factors, link strains, pair lists, time -- in either precision, whatever the calls
+are cut into.  Only the centre of mass is summed in another order."""
+import numpy as np
+import pytest
+
+from gpuvoxels_amd import _abi, engine, workloads
+from gpuvoxels_amd.model import Ext, MT
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac", "strain", "max_strain", "small_angle")
+
+
+def run(models, chunks, noalloc, precision, interval=0, table=0, graph=1, path=_abi.PATH_STREAM):
+    b = engine.Batch(precision=precision, path=path, collision_rebuild_interval=interval, collision_table_entries=table, use_graph=graph)
+    slots = [b.admit(m) for m in models]
+    for n in chunks:
+        target = None
+        while True:   # a simulation that stood still for a table catches up after the poll
+            st = b.poll()
+            if target is None:
+                target = [st[s].steps + n for s in slots]
+            lag = max((t - st[s].steps for t, s in zip(target, slots) if st[s].state == _abi.SIM_RUNNING), default=0)
+            if lag <= 0:
+                break
+            (b.step_noalloc if noalloc else b.step)(min(n, lag))
+    st = b.poll()
+    out = []
+    for m, s in zip(models, slots):
+        nl = len(engine.topology(m)[0])
+        out.append((b.read_state(s, nl=max(nl, 1)), b.collision_pairs(s) if m.collisions_enabled else None, st[s]))
+    b.close()
+    return out
+
+
+def assert_equal(a, c):
+    for (x, px, sx), (y, py, sy) in zip(a, c):
+        assert sx.steps == sy.steps and sx.state == sy.state and sx.current_time == sy.current_time
+        for k in KEYS:
+            assert np.array_equal(x[k], y[k], equal_nan=True), k
+        if px is not None:
+            assert np.array_equal(px, py)
+
+
+def varied():
+    """Odd sizes, several phases, externals on edges and inside, fixed and failing and
+    plastic materials, several simulations in a batch."""
+    plate = workloads.slab(19, 11, 5, steps=0, collisions=False)
+    plate.externals = [Ext(voxel=0, dof_fixed=63, translate=(0.0, 0.0, 0.001), rotate=(0.0, 0.1, 0.0)),
+                       Ext(voxel=40, dof_fixed=5, force=(0.0, 0.02, 0.0)), Ext(voxel=500, dof_fixed=8, moment=(1e-5, 0.0, 0.0))]
+    bot = workloads.robot(np.random.default_rng(3), grid=13, steps=0)
+    bot.materials[1].fixed = 1
+    bot.materials[2].mat_model, bot.materials[2].fail_stress = _abi.MDL_LINEAR_FAIL, 800.0
+    bot.phase = np.round(np.random.default_rng(4).random(bot.n_voxels) * 30) / 30.0
+    line = workloads.cube(2, steps=0)
+    line.ijk = np.stack([np.arange(700), np.zeros(700, int), np.zeros(700, int)], 1).astype(np.int32)
+    line.mat, line.phase = np.zeros(700, np.int32), np.linspace(0, 1, 700).round(1)
+    line.volume_effects = 0
+    return [plate, bot, line, workloads.cube(3, steps=0)]
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+@pytest.mark.parametrize("chunks", [[5], [6], [97, 6, 5, 64], [97, 4, 3, 64], [1, 33, 200]])
+def test_equals_step_kernels(precision, chunks):
+    models = varied()
+    assert_equal(run(models, chunks, False, precision), run(models, chunks, True, precision))
+
+
+def test_equals_step_kernels_large_angles_and_divergence():
+    """A robot flung apart: large-angle links, then a diverged one (the same step)."""
+    models = varied()[:2]
+    rng = np.random.default_rng(8)
+    models[0].init_velocity = rng.normal(0, 4.0, (models[0].n_voxels, 3))
+    models[1].init_velocity = rng.normal(0, 300.0, (models[1].n_voxels, 3))
+    a, c = (run(models, [150, 150], k, _abi.PREC_F64) for k in (False, True))
+    assert a[1][2].state == _abi.SIM_DIVERGED and np.any(a[0][0]["small_angle"] == 0)
+    assert_equal(a, c)
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+@pytest.mark.parametrize("count,radius,arena,interval,table", [(9, 4, 26, 8, 0), (30, 2, 24, 0, 0), (14, 3, 26, 5, 16)])
+def test_collisions_equal_step_kernels(precision, count, radius, arena, interval, table):
+    """Touching balls: several to a tile, one to a tile; lists rebuilt when stale and
+    periodically; a table that has to grow."""
+    m = workloads.arena_balls(count, radius=radius, arena=arena, gap=0.0, sigma_v=0.4, steps=0, seed=5)
+    drop = workloads.drop(9, gap=1, shift=2, steps=0)      # two bodies of several tiles each
+    models = [m, drop]
+    chunks = [120, 1, 7, 240]
+    a = run(models, chunks, False, precision, interval, table)
+    assert_equal(a, run(models, chunks, True, precision, interval, 0))
+    assert len(a[0][1]) > 0
+
+
+def test_long_partner_lists():
+    """Two plates pressed face to face within the watch radius: every voxel of the faces
+    watches more partners than its LDS column holds."""
+    m = workloads.drop(4, gap=1, shift=0, steps=0)
+    z, y, x = np.meshgrid(np.arange(1), np.arange(16), np.arange(16), indexing="ij")
+    a = np.stack([x.ravel(), y.ravel(), z.ravel()], 1)
+    cells = np.concatenate([a, a + [0, 0, 2]])
+    m.ijk = cells[np.lexsort((cells[:, 0], cells[:, 1], cells[:, 2]))].astype(np.int32)
+    m.mat, m.phase = np.zeros(len(cells), np.int32), None
+    m.watch_distance = 3.5
+    a, c = (run([m], [40], k, _abi.PREC_F64) for k in (False, True))
+    assert len(a[0][1]) > 512 * 24 // 2
+    assert_equal(a, c)
+
+
+def test_wide_link_hop_radius():
+    """A watch distance whose nearby radius is beyond the lattice masks (sorted lists)."""
+    m = workloads.slab(12, 11, 4, steps=0, collisions=True)
+    m.watch_distance = 2.0
+    a, c = (run([m], [30, 30], k, _abi.PREC_F64) for k in (False, True))
+    assert_equal(a, c)
+
+
+def test_stop_conditions_and_no_graph():
+    models = varied()[:2]
+    models[0].stop_tokens = [(MT["mtCONST"], 0.004), (MT["mtVAR"], 4.0), (MT["mtGREATERTHAN"], 0.0), (MT["mtEND"], 0.0)]
+    models[1].max_steps = 77
+    a = run(models, [150], False, _abi.PREC_F64, graph=0)
+    c = run(models, [150], True, _abi.PREC_F64)
+    assert all(x[2].state == _abi.SIM_DONE for x in a)
+    assert_equal(a, c)
+
+
+def test_beside_resident_and_retired():
+    """One batch with one-workgroup and fused simulations, one of the latter retired and
+    replaced: each ends as alone."""
+    big = workloads.drop(9, gap=1, shift=2, steps=0)
+    other = workloads.slab(21, 10, 6, steps=0, collisions=True)
+    small = workloads.robots(2, seed=6, grid=8, steps=0)
+    b = engine.Batch(precision=_abi.PREC_F64, path=_abi.PATH_AUTO)
+    s = [b.admit(m) for m in (big, small[0], other, small[1])]
+    assert b.workgroups(s[0]) == 0 and b.workgroups(s[2]) == 0
+    b.step(90)
+    b.retire(s[0])
+    again = b.admit(big)
+    b.step(90)
+    for slot, m, n in ((s[2], other, 180), (again, big, 90), (s[3], small[1], 180)):
+        ref = run([m], [n], True, _abi.PREC_F64)[0][0]
+        got = b.read_state(slot)
+        for k in ("pos", "orient", "lin_mom", "ang_mom", "flags"):
+            assert np.array_equal(got[k], ref[k]), k
+    b.close()
