@@ -57,5 +57,8 @@ void launchDt(const DevBatch<double>& b, hipStream_t s, int s0, int s1);
 // stride dstFs), in the state precision
 void launchCopyLoads(const DevBatch<float>& b, hipStream_t s, const void* src, size_t srcFs, void* dst, size_t dstFs, int nv);
 void launchCopyLoads(const DevBatch<double>& b, hipStream_t s, const void* src, size_t srcFs, void* dst, size_t dstFs, int nv);
+// writes the state of the pieces jobs[0, n) to out (both in pinned host memory)
+void launchPull(const DevBatch<float>& b, hipStream_t s, const PullJob* jobs, int n, char* out);
+void launchPull(const DevBatch<double>& b, hipStream_t s, const PullJob* jobs, int n, char* out);
 }  // namespace vx3
 #endif

@@ -52,6 +52,10 @@ void launchStep(const DevBatch<VX_REAL>& b, hipStream_t s, const StepOpts& o, hi
 #undef VX3_EV
 }
 
+void launchPull(const DevBatch<VX_REAL>& b, hipStream_t s, const PullJob* jobs, int n, char* out) {
+    if (n > 0) hipLaunchKernelGGL(VX_NS::k_pull, dim3(n), dim3(VX3_PULL_PIECE), 0, s, b, jobs, out);
+}
+
 void launchCopyLoads(const DevBatch<VX_REAL>& b, hipStream_t s, const void* src, size_t srcFs, void* dst, size_t dstFs, int nv) {
     if (nv > 0)
         hipLaunchKernelGGL(VX_NS::k_copy_loads, dim3((nv + 255) / 256), dim3(256), 0, s, (const VX_REAL*)src, srcFs,

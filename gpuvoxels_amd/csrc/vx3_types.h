@@ -249,6 +249,21 @@ struct TsAux {                       // per tile, by parity of the step that wri
     double part[2][4];               // centre-of-mass partial sums
 };
 
+// Up to VX3_PULL_PIECE voxels or links of one simulation whose state the host reads (k_pull): at
+// `off` of the output a word with the simulation's flags, from VX3_PULL_HEAD on the parts asked
+// for, in the order of their bits: doubles, then ints.
+struct PullJob {
+    int slot, first, n, parts;       // batch index of the first one
+    long long off;
+    int owner;                       // the caller's
+};
+#define VX3_PULL_PIECE 256
+#define VX3_PULL_HEAD 16
+enum {
+    PULL_POS = 1, PULL_LIN = 2, PULL_ANG = 4, PULL_ORIENT = 8, PULL_TEMP = 16, PULL_INIT = 32,   // per voxel: 3, 3, 3, 4, 1, 3
+    PULL_STRAIN = 64, PULL_MAXSTRAIN = 128,                                                      // per link
+    PULL_FLAGS = 256, PULL_LFLAGS = 512                                                          // ints, per voxel and per link
+};
 // One tile of a simulation that the resident kernel runs on several workgroups (tiled
 // launch): the tile owns a compact block of the simulation's voxels and computes every
 // link with an end among them; the other ends (its halo) are read from the exchange

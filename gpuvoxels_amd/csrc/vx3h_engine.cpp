@@ -465,16 +465,56 @@ vx3h_status copyReal(vx3h_batch* b, void* dst, const std::vector<double>& src) {
     return VX3H_OK;
 }
 
-vx3h_status readReal(vx3h_batch* b, const void* src, size_t n, std::vector<double>& out) {
-    out.resize(n);
-    if (b->realSize == 4) {
-        std::vector<float> t(n);
-        HIPCHK(hipMemcpy(t.data(), src, n * 4, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < n; i++) out[i] = t[i];
-    } else {
-        HIPCHK(hipMemcpy(out.data(), src, n * 8, hipMemcpyDeviceToHost));
+// The most that one launch of k_pull writes: two such regions of the staging buffer, one being
+// written while the host copies the other out.
+constexpr size_t PULL_REGION = (size_t)4 << 20;
+
+size_t pullBytes(const PullJob& j) {
+    const int p = j.parts;
+    const size_t d = 3 * (!!(p & PULL_POS) + !!(p & PULL_LIN) + !!(p & PULL_ANG) + !!(p & PULL_INIT)) + 4 * !!(p & PULL_ORIENT) +
+                     !!(p & PULL_TEMP) + !!(p & PULL_STRAIN) + !!(p & PULL_MAXSTRAIN);
+    const size_t i = !!(p & PULL_FLAGS) + !!(p & PULL_LFLAGS);
+    return (VX3_PULL_HEAD + (8 * d + 4 * i) * j.n + 15) & ~(size_t)15;
+}
+
+// `n` elements from batch index `first` on, in pieces
+void pullAdd(std::vector<PullJob>& jobs, int slot, int first, int n, int parts, int owner = 0) {
+    for (int i = 0; i < n; i += VX3_PULL_PIECE) jobs.push_back({slot, first + i, std::min(n - i, VX3_PULL_PIECE), parts, 0, owner});
+}
+
+// Reads the pieces' state: take(piece, its output) for each, in order.  The main stream's work
+// is done first.
+template <typename F> vx3h_status pullState(vx3h_batch* b, std::vector<PullJob>& jobs, F take) {
+    if (jobs.empty()) return VX3H_OK;
+    std::vector<size_t> first;   // per launch its first piece
+    size_t used = PULL_REGION, most = 0;
+    for (size_t i = 0; i < jobs.size(); i++) {
+        const size_t r = pullBytes(jobs[i]);
+        if (used + r > PULL_REGION) { first.push_back(i); used = 0; }
+        jobs[i].off = (long long)(used + (first.size() & 1 ? 0 : PULL_REGION));
+        used += r;
+        most = std::max(most, used);
     }
-    return VX3H_OK;
+    const size_t launches = first.size();
+    first.push_back(jobs.size());
+    const size_t region = launches > 1 ? 2 * PULL_REGION : (most + 255) & ~(size_t)255;
+    char* base;
+    if (vx3h_status st = stageAlloc(b, region + jobs.size() * sizeof(PullJob), &base)) return st;
+    PullJob* list = (PullJob*)(base + region);
+    memcpy(list, jobs.data(), jobs.size() * sizeof(PullJob));
+    auto launch = [&](size_t k) -> vx3h_status {
+        if (b->realSize == 4) launchPull(b->db, b->stream, list + first[k], (int)(first[k + 1] - first[k]), base);
+        else launchPull(*reinterpret_cast<DevBatch<double>*>(&b->db), b->stream, list + first[k], (int)(first[k + 1] - first[k]), base);
+        HIPCHK(hipGetLastError());
+        return VX3H_OK;
+    };
+    vx3h_status st = launch(0);
+    for (size_t k = 0; k < launches && !st; k++) {
+        HIPCHK(hipStreamSynchronize(b->stream));
+        if (k + 1 < launches) st = launch(k + 1);
+        for (size_t i = first[k]; i < first[k + 1]; i++) take(jobs[i], base + jobs[i].off);
+    }
+    return st;
 }
 
 char* at(void* base, size_t elem, size_t idx) { return (char*)base + elem * idx; }
@@ -2040,7 +2080,13 @@ extern "C" vx3h_status vx3h_batch_sync(vx3h_batch* b) {
 }
 
 namespace vx3 {
-vx3h_status pollOne(vx3h_batch* b, int s, const SimCtl& c, vx3h_sim_status& o, std::vector<double>* posOut) {
+// Sums over a simulation's measured voxels, in voxel order.
+struct PollSums {
+    double tot = 0, x = 0, y = 0, z = 0, dist = 0;
+    int n = 0;
+};
+
+void pollStatus(const vx3h_batch* b, int s, const SimCtl& c, const PollSums& m, vx3h_sim_status& o) {
     const SlotHost& sh = b->slots[s];
     memset(&o, 0, sizeof(o));
     o.slot = s;
@@ -2055,46 +2101,46 @@ vx3h_status pollOne(vx3h_batch* b, int s, const SimCtl& c, vx3h_sim_status& o, s
     o.recent_angle = c.recentAngle;
     // initial center of mass and positions: the admission's, or a secondary experiment's reset
     for (int k = 0; k < 3; k++) o.initial_com[k] = c.com0[k];
-    std::vector<double> x, y, z;
-    vx3h_status st;
-    const size_t rs = b->realSize;
-    if ((st = readReal(b, at(b->db.px, rs, sh.v0), sh.nv, x))) return st;
-    if ((st = readReal(b, at(b->db.py, rs, sh.v0), sh.nv, y))) return st;
-    if ((st = readReal(b, at(b->db.pz, rs, sh.v0), sh.nv, z))) return st;
-    std::vector<double> ip;
-    if (c.flags & SC_SECONDARY) {
-        ip.resize(3 * (size_t)sh.nv);
-        for (int k = 0; k < 3; k++)
-            HIPCHK(hipMemcpy(ip.data() + (size_t)k * sh.nv, b->db.ip + (size_t)k * b->db.Vcap + sh.v0, sh.nv * 8, hipMemcpyDeviceToHost));
-    }
-    // updateCurrentCenterOfMass (VX3_VoxelyzeKernel.cu:477-493) + collectResults totals (VX3_SimulationManager.cu:442-452)
-    double tot = 0, sx = 0, sy = 0, sz = 0, dist = 0;
-    int nm = 0;
-    for (int i = 0; i < sh.nv; i++) {
-        if (!sh.measured[i]) continue;
-        double m = sh.mass[i];
-        sx += x[i] * m; sy += y[i] * m; sz += z[i] * m;
-        tot += m;
-        nm++;
-        const double ix = ip.empty() ? sh.ijk[3 * i] * sh.voxSize : ip[i];
-        const double iy = ip.empty() ? sh.ijk[3 * i + 1] * sh.voxSize : ip[sh.nv + i];
-        const double iz = ip.empty() ? sh.ijk[3 * i + 2] * sh.voxSize : ip[2 * (size_t)sh.nv + i];
-        double dx = x[i] - ix, dy = y[i] - iy, dz = z[i] - iz;
-        dist += sqrt(dx * dx + dy * dy + dz * dz);
-    }
-    if (tot != 0) { double inv = 1.0 / tot; o.current_com[0] = inv * sx; o.current_com[1] = inv * sy; o.current_com[2] = inv * sz; }
-    o.num_measured_voxel = nm;
-    o.total_distance_of_all_voxels = dist;
+    if (m.tot != 0) { double inv = 1.0 / m.tot; o.current_com[0] = inv * m.x; o.current_com[1] = inv * m.y; o.current_com[2] = inv * m.z; }
+    o.num_measured_voxel = m.n;
+    o.total_distance_of_all_voxels = m.dist;
     double off[3] = {o.current_com[0] - c.com0[0], o.current_com[1] - c.com0[1], o.current_com[2] - c.com0[2]};
     // computeFitness (VX3_VoxelyzeKernel.cu:530-534)
     o.num_close_pairs = c.closePairs;
     o.target_closeness = c.closeness;
     o.fitness = evalMathTree(sh.fit.data(), (int)sh.fit.size(), off[0], off[1], off[2], c.hits, c.t, c.recentAngle, c.closeness,
                              c.closePairs, sh.nv);
-    if (posOut) {
-        posOut->resize(3 * sh.nv);
-        for (int i = 0; i < sh.nv; i++) { (*posOut)[3 * i] = x[i]; (*posOut)[3 * i + 1] = y[i]; (*posOut)[3 * i + 2] = z[i]; }
+}
+
+// The statuses of simulations `slots`, whose positions are read in one go.
+vx3h_status pollSlots(vx3h_batch* b, const std::vector<int>& slots, const std::vector<SimCtl>& ctl, vx3h_sim_status* out) {
+    std::vector<PullJob> jobs;
+    for (size_t i = 0; i < slots.size(); i++) {
+        const SlotHost& sh = b->slots[slots[i]];
+        pullAdd(jobs, slots[i], sh.v0, sh.nv, PULL_POS | (ctl[slots[i]].flags & SC_SECONDARY ? PULL_INIT : 0), (int)i);
     }
+    std::vector<PollSums> sums(slots.size());
+    // updateCurrentCenterOfMass (VX3_VoxelyzeKernel.cu:477-493) + collectResults totals (VX3_SimulationManager.cu:442-452)
+    vx3h_status st = pullState(b, jobs, [&](const PullJob& j, const char* at) {
+        const SlotHost& sh = b->slots[j.slot];
+        PollSums& m = sums[j.owner];
+        const double *p = (const double*)(at + VX3_PULL_HEAD), *ip = j.parts & PULL_INIT ? p + 3 * j.n : nullptr;
+        for (int k = 0; k < j.n; k++, p += 3) {
+            const int i = j.first - sh.v0 + k;
+            if (!sh.measured[i]) continue;
+            const double mass = sh.mass[i];
+            m.x += p[0] * mass; m.y += p[1] * mass; m.z += p[2] * mass;
+            m.tot += mass;
+            m.n++;
+            const double ix = ip ? ip[3 * k] : sh.ijk[3 * i] * sh.voxSize;
+            const double iy = ip ? ip[3 * k + 1] : sh.ijk[3 * i + 1] * sh.voxSize;
+            const double iz = ip ? ip[3 * k + 2] : sh.ijk[3 * i + 2] * sh.voxSize;
+            const double dx = p[0] - ix, dy = p[1] - iy, dz = p[2] - iz;
+            m.dist += sqrt(dx * dx + dy * dy + dz * dz);
+        }
+    });
+    if (st) return st;
+    for (size_t i = 0; i < slots.size(); i++) pollStatus(b, slots[i], ctl[slots[i]], sums[i], out[i]);
     return VX3H_OK;
 }
 }  // namespace vx3
@@ -2226,13 +2272,11 @@ vx3h_status pollFinished(vx3h_batch* b, std::vector<vx3h_sim_status>& finished) 
         vx3h_status gs = growCollisionTables(b, ctl);
         if (gs) return gs;
     }
-    for (int s = 0; s < (int)b->slots.size(); s++) {
-        if (!b->slots[s].used || ctl[s].state == VX3H_SIM_RUNNING) continue;
-        finished.emplace_back();
-        vx3h_status st = pollOne(b, s, ctl[s], finished.back(), nullptr);
-        if (st) return st;
-    }
-    return VX3H_OK;
+    std::vector<int> slots;
+    for (int s = 0; s < (int)b->slots.size(); s++)
+        if (b->slots[s].used && ctl[s].state != VX3H_SIM_RUNNING) slots.push_back(s);
+    finished.resize(slots.size());
+    return pollSlots(b, slots, ctl, finished.data());
 }
 }  // namespace vx3
 
@@ -2240,21 +2284,21 @@ extern "C" vx3h_status vx3h_batch_poll(vx3h_batch* b, vx3h_sim_status* out, int 
     if (!b || !n) FAILV(VX3H_EINVAL, "null argument");
     HIPCHK(hipSetDevice(b->device));
     HIPCHK(hipStreamSynchronize(b->stream));
+    const bool grow = b->anyColl || b->anyAttach;
     std::vector<SimCtl> ctl(b->slots.size());
-    if (!ctl.empty()) HIPCHK(hipMemcpy(ctl.data(), b->db.sims, ctl.size() * sizeof(SimCtl), hipMemcpyDeviceToHost));
-    if (b->anyColl || b->anyAttach) {
+    if (!ctl.empty() && (out || grow)) HIPCHK(hipMemcpy(ctl.data(), b->db.sims, ctl.size() * sizeof(SimCtl), hipMemcpyDeviceToHost));
+    if (grow) {
         vx3h_status gs = growCollisionTables(b, ctl);
         if (gs) return gs;
     }
+    std::vector<int> slots;
     int k = 0;
     for (int s = 0; s < (int)b->slots.size(); s++) {
         if (!b->slots[s].used) continue;
-        if (out && k < cap) {
-            vx3h_status st = pollOne(b, s, ctl[s], out[k], nullptr);
-            if (st) return st;
-        }
+        if (out && k < cap) slots.push_back(s);
         k++;
     }
+    if (vx3h_status st = pollSlots(b, slots, ctl, out)) return st;
     *n = k;
     return VX3H_OK;
 }
@@ -2385,65 +2429,39 @@ extern "C" vx3h_status vx3h_sim_read_state(vx3h_batch* b, int slot, vx3h_state_v
     const SlotHost& sh = b->slots[slot];
     // links written: the admitted ones, or with a capacity also those attach made
     const int nlOut = view->link_capacity > 0 ? std::min(view->link_capacity, sh.nlSeen) : sh.nl;
-    const DevBatch<float>& d = b->db;
-    const size_t rs = b->realSize;
-    std::vector<double> t0, t1, t2, t3;
-    vx3h_status st;
-    auto get3 = [&](void* a, void* bb, void* c, double* out) -> vx3h_status {
-        vx3h_status s2;
-        if ((s2 = readReal(b, at(a, rs, sh.v0), sh.nv, t0))) return s2;
-        if ((s2 = readReal(b, at(bb, rs, sh.v0), sh.nv, t1))) return s2;
-        if ((s2 = readReal(b, at(c, rs, sh.v0), sh.nv, t2))) return s2;
-        for (int i = 0; i < sh.nv; i++) { out[3 * i] = t0[i]; out[3 * i + 1] = t1[i]; out[3 * i + 2] = t2[i]; }
-        return VX3H_OK;
-    };
-    if (view->pos && (st = get3(d.px, d.py, d.pz, view->pos))) return st;
-    if (view->lin_mom && (st = get3(d.mx, d.my, d.mz, view->lin_mom))) return st;
-    if (view->ang_mom && (st = get3(d.ax, d.ay, d.az, view->ang_mom))) return st;
-    if (view->orient) {
-        if ((st = readReal(b, at(d.ow, rs, sh.v0), sh.nv, t3))) return st;
-        if ((st = readReal(b, at(d.ox, rs, sh.v0), sh.nv, t0))) return st;
-        if ((st = readReal(b, at(d.oy, rs, sh.v0), sh.nv, t1))) return st;
-        if ((st = readReal(b, at(d.oz, rs, sh.v0), sh.nv, t2))) return st;
-        for (int i = 0; i < sh.nv; i++) {
-            view->orient[4 * i] = t3[i]; view->orient[4 * i + 1] = t0[i]; view->orient[4 * i + 2] = t1[i]; view->orient[4 * i + 3] = t2[i];
-        }
-    }
-    if (view->vox_flags) HIPCHK(hipMemcpy(view->vox_flags, d.vflags + sh.v0, sh.nv * 4, hipMemcpyDeviceToHost));
-    if (view->init_pos) {
-        SimCtl c;
-        HIPCHK(hipMemcpy(&c, b->db.sims + slot, sizeof(SimCtl), hipMemcpyDeviceToHost));
-        std::vector<double> col(sh.nv);
-        for (int k = 0; k < 3; k++) {
-            if (c.flags & SC_SECONDARY)
-                HIPCHK(hipMemcpy(col.data(), d.ip + (size_t)k * d.Vcap + sh.v0, sh.nv * 8, hipMemcpyDeviceToHost));
-            else
-                for (int i = 0; i < sh.nv; i++) col[i] = sh.ijk[3 * i + k] * sh.voxSize;
-            for (int i = 0; i < sh.nv; i++) view->init_pos[3 * i + k] = col[i];
-        }
-    }
-    if (view->temp) {
-        std::vector<float> tf(sh.nv);
-        HIPCHK(hipMemcpy(tf.data(), d.tfac + sh.v0, sh.nv * 4, hipMemcpyDeviceToHost));
-        for (int i = 0; i < sh.nv; i++) view->temp[i] = tf[i];   // thermal size factor 1 + T*CTE
-    }
-    if (nlOut && (view->link_strain || view->link_max_strain)) {
-        std::vector<float> a(nlOut);
-        if (view->link_strain) {
-            HIPCHK(hipMemcpy(a.data(), d.strain + sh.l0, nlOut * 4, hipMemcpyDeviceToHost));
-            for (int i = 0; i < nlOut; i++) view->link_strain[i] = a[i];
-        }
-        if (view->link_max_strain) {
-            HIPCHK(hipMemcpy(a.data(), d.maxStrain + sh.l0, nlOut * 4, hipMemcpyDeviceToHost));
-            for (int i = 0; i < nlOut; i++) view->link_max_strain[i] = a[i];
-        }
-    }
-    if (nlOut && view->link_small_angle) {
-        std::vector<int> f(nlOut);
-        HIPCHK(hipMemcpy(f.data(), d.lflags + sh.l0, nlOut * 4, hipMemcpyDeviceToHost));
-        for (int i = 0; i < nlOut; i++) view->link_small_angle[i] = (f[i] & LF_SMALL_ANGLE) ? 1 : 0;
-    }
-    return VX3H_OK;
+    std::vector<PullJob> jobs;
+    const int voxels = (view->pos ? PULL_POS : 0) | (view->lin_mom ? PULL_LIN : 0) | (view->ang_mom ? PULL_ANG : 0) |
+                       (view->orient ? PULL_ORIENT : 0) | (view->temp ? PULL_TEMP : 0) | (view->init_pos ? PULL_INIT : 0) |
+                       (view->vox_flags ? PULL_FLAGS : 0);
+    const int links = (view->link_strain ? PULL_STRAIN : 0) | (view->link_max_strain ? PULL_MAXSTRAIN : 0) |
+                      (view->link_small_angle ? PULL_LFLAGS : 0);
+    if (voxels) pullAdd(jobs, slot, sh.v0, sh.nv, voxels);
+    if (links) pullAdd(jobs, slot, sh.l0, nlOut, links, 1);
+    return pullState(b, jobs, [&](const PullJob& j, const char* at) {
+        const bool secondary = (*(const int*)at & SC_SECONDARY) != 0;
+        const size_t first = j.first - (j.owner ? sh.l0 : sh.v0), n = j.n;
+        const double* d = (const double*)(at + VX3_PULL_HEAD);
+        auto rows = [&](int part, double* out, size_t per) {
+            if (!(j.parts & part)) return;
+            memcpy(out + first * per, d, n * per * sizeof(double));
+            d += n * per;
+        };
+        rows(PULL_POS, view->pos, 3);
+        rows(PULL_LIN, view->lin_mom, 3);
+        rows(PULL_ANG, view->ang_mom, 3);
+        rows(PULL_ORIENT, view->orient, 4);
+        rows(PULL_TEMP, view->temp, 1);   // thermal size factor 1 + T*CTE
+        if ((j.parts & PULL_INIT) && !secondary) {
+            for (size_t i = 3 * first; i < 3 * (first + n); i++) view->init_pos[i] = sh.ijk[i] * sh.voxSize;
+            d += 3 * n;
+        } else rows(PULL_INIT, view->init_pos, 3);
+        rows(PULL_STRAIN, view->link_strain, 1);
+        rows(PULL_MAXSTRAIN, view->link_max_strain, 1);
+        const int* w = (const int*)d;
+        if (j.parts & PULL_FLAGS) memcpy(view->vox_flags + first, w, n * sizeof(int));
+        if (j.parts & PULL_LFLAGS)
+            for (size_t i = 0; i < n; i++) view->link_small_angle[first + i] = (w[i] & LF_SMALL_ANGLE) ? 1 : 0;
+    });
 }
 
 namespace {
