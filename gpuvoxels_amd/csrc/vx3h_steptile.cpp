@@ -140,7 +140,14 @@ bool planStepTiles(int nv, const int* ijk, int nl, const int* lneg, const int* l
         size_t surface = 0;
         if (n <= VX3_TS_OWN) for (size_t j = 0; j < n; j++) surface += !interior[b[j]];
         if (n > VX3_TS_OWN || surface > VX3_TS_BLOCK) {
-            std::sort(b, b + n);
+            // ascending; a body's voxels mostly have all indices of their range
+            int lo = INT_MAX, hi = 0;
+            for (size_t j = 0; j < n; j++) { lo = std::min(lo, b[j]); hi = std::max(hi, b[j]); }
+            if ((size_t)(hi - lo) < 4 * n) {
+                for (size_t j = 0; j < n; j++) seen[b[j]] = 2;
+                size_t j = 0;
+                for (int v = lo; v <= hi; v++) if (seen[v] == 2) { b[j++] = v; seen[v] = 1; }
+            } else std::sort(b, b + n);
             items.resize(n);
             for (size_t j = 0; j < n; j++) items[j] = {b[j], {ijk[3 * (size_t)b[j]], ijk[3 * (size_t)b[j] + 1], ijk[3 * (size_t)b[j] + 2]}};
             c.cut(items.data(), n, (int)((n + VX3_TS_CUT - 1) / VX3_TS_CUT));
@@ -205,12 +212,14 @@ bool planStepTiles(int nv, const int* ijk, int nl, const int* lneg, const int* l
     const int T = (int)c.parts.size();
     if (T > (INT_MAX >> VX3_TS_SLOT_BITS)) return false;
     std::vector<int> place(nv), hslot(nv, -1), touched;
+    std::vector<std::pair<uint64_t, int>> keys;
     for (int t = 0; t < T; t++) {
         std::vector<int>& p = c.parts[t];
         // the surface first, body by body: a list rebuild bounds each 64 of a tile's surface voxels
-        std::sort(p.begin(), p.end(), [&](int x, int y) {
-            return interior[x] != interior[y] ? interior[x] < interior[y] : body[x] != body[y] ? body[x] < body[y] : x < y;
-        });
+        keys.resize(p.size());
+        for (size_t i = 0; i < p.size(); i++) keys[i] = {(uint64_t)(interior[p[i]] != 0) << 32 | (uint32_t)body[p[i]], p[i]};
+        std::sort(keys.begin(), keys.end());
+        for (size_t i = 0; i < p.size(); i++) p[i] = keys[i].second;
         for (size_t i = 0; i < p.size(); i++) place[p[i]] = t << VX3_TS_SLOT_BITS | (int)i;
     }
     auto tileOf = [&](int v) { return place[v] >> VX3_TS_SLOT_BITS; };
