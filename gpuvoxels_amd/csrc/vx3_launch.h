@@ -37,6 +37,18 @@ hipError_t launchResident(const DevBatch<float>& b, hipStream_t s, int shape, bo
                           int nSteps, hipEvent_t* ev = nullptr);
 hipError_t launchResident(const DevBatch<double>& b, hipStream_t s, int shape, bool collisions, const int* simList, int nSims,
                           int nSteps, hipEvent_t* ev = nullptr);
+// Shapes of the one-workgroup kernel that computes the links of all axes at once (no
+// collisions): block, link slots.  A sim fits when V <= block and it has <= links links.
+struct ResidentAllInfo { int block, links; };
+int residentAllShapes(const DevBatch<float>& b, ResidentAllInfo* out, int cap);
+int residentAllShapes(const DevBatch<double>& b, ResidentAllInfo* out, int cap);
+hipError_t launchResidentAll(const DevBatch<float>& b, hipStream_t s, int shape, const int* simList, int nSims, int nSteps,
+                             hipEvent_t* ev = nullptr);
+hipError_t launchResidentAll(const DevBatch<double>& b, hipStream_t s, int shape, const int* simList, int nSims, int nSteps,
+                             hipEvent_t* ev = nullptr);
+// workgroups of shape `shape`'s kernel without collisions that one compute unit holds at once
+hipError_t residentOccupancy(const DevBatch<float>& b, int shape, int* perCU);
+hipError_t residentOccupancy(const DevBatch<double>& b, int shape, int* perCU);
 // Launches the tiled resident kernel of shape `shape` (no collisions) over the tiles
 // ta.tiles[0, nTiles) after clearing ta.sync[0, nSync); every tile is resident at once.
 hipError_t launchTiled(const DevBatch<float>& b, hipStream_t s, int shape, const TileArgs& ta, int nTiles, int nSync,

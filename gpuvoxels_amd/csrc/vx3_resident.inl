@@ -50,6 +50,9 @@
 // simulation placed in a tiled launch) has no barrier or exchange and steps exactly as
 // the one-workgroup kernel does.
 //
+// Small simulations without collisions whose links' loads fit LDS all at once run k_resident_all
+// (vx3_resident_all.inl) instead.
+//
 // Included by the per-precision kernel units after vx3_kernels.inl (VX_NS, real).
 
 namespace vx3 {

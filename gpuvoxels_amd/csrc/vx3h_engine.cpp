@@ -195,6 +195,10 @@ struct vx3h_batch {
     std::vector<ResidentShapeInfo> shapes;
     std::vector<int> shapePref;                  // shape indices in preference order
     std::vector<std::vector<int>> resLists;
+    std::vector<std::vector<int>> launchLists;   // the same as the launches take them (syncResLists)
+    std::vector<ResidentAllInfo> allShapes;
+    std::vector<int> resPerCU;                   // per shape, workgroups that a compute unit holds
+    int cus = 0;
     std::vector<int*> dResLists;
     std::vector<size_t> capRes;
     bool resDirty = false;
@@ -577,10 +581,44 @@ vx3h_status ensureGraph(vx3h_batch* b, int steps, int solo) {
     return VX3H_OK;
 }
 
+// Which kernel the one-workgroup simulations without collisions take.  The one with the links
+// of all axes at once has the shorter step (see k_resident_all) but holds a compute unit by
+// itself, so it is taken where each simulation has one anyway: when they are no more than the
+// units, each in its smallest shape, or when the axis-by-axis shapes they would take hold a
+// unit each too, all in one shape (workgroups go round the chip's eight dies kernel by kernel,
+// so two kernels' remainders can leave one die a round more: 512 robots in FP32, 23.5 us a step
+// in two shapes, 17.1 in one, 22.4 axis by axis).  Past that line more workgroups a unit win:
+// 300 robots on 10^3 grids, FP32, 11.5 us a step axis by axis, 17.2 here; 512, 13.6 and 18.7.
 vx3h_status syncResLists(vx3h_batch* b) {
     if (!b->resDirty) return VX3H_OK;
-    for (size_t i = 0; i < b->resLists.size(); i++) {
-        const auto& L = b->resLists[i];
+    const size_t ns = b->shapes.size(), na = b->allShapes.size();
+    b->launchLists = b->resLists;
+    b->launchLists.resize(2 * ns + na);
+    size_t total = 0;
+    bool alone = true;   // every kernel of the lists holds a compute unit
+    for (size_t i = 0; i < ns; i++) {
+        total += b->resLists[i].size();
+        alone = alone && (b->resLists[i].empty() || b->resPerCU[i] <= 1);
+    }
+    // (a configured block size asks for the shapes of that size)
+    if (b->cfg.block_size == 0 && (alone || total <= (size_t)b->cus)) {
+        auto fits = [&](int s, size_t j) { return b->slots[s].nv <= b->allShapes[j].block && b->slots[s].nl <= b->allShapes[j].links; };
+        size_t one = 0;   // the shape that all of them fit
+        for (size_t i = 0; i < ns; i++)
+            for (int s : b->resLists[i])
+                while (one < na && !fits(s, one)) one++;
+        const bool few = total <= (size_t)b->cus;
+        for (size_t i = 0; i < ns && (few || one < na); i++) {
+            b->launchLists[i].clear();
+            for (int s : b->resLists[i]) {
+                size_t j = few ? 0 : one;
+                while (j < na && !fits(s, j)) j++;
+                b->launchLists[j < na ? 2 * ns + j : i].push_back(s);
+            }
+        }
+    }
+    for (size_t i = 0; i < b->launchLists.size(); i++) {
+        const auto& L = b->launchLists[i];
         if (L.empty()) continue;
         if (L.size() > b->capRes[i]) {
             if (b->dResLists[i]) HIPCHK(hipFree(b->dResLists[i]));
@@ -592,6 +630,9 @@ vx3h_status syncResLists(vx3h_batch* b) {
     b->resDirty = false;
     return VX3H_OK;
 }
+
+// list i of launchLists holds simulations without collisions
+bool absorbable(const vx3h_batch* b, size_t i) { return i < b->shapes.size() || i >= 2 * b->shapes.size(); }
 
 // grows a device array to at least n elements (contents not kept)
 template <typename T> vx3h_status growDev(T** p, size_t* cap, size_t n) {
@@ -900,9 +941,9 @@ vx3h_status launchResidentAll(vx3h_batch* b, int nSteps, hipEvent_t* ev) {
     vx3h_status st = syncResLists(b);
     if (st || (st = syncTiles(b))) return st;
     bool forked = false;
-    for (size_t i = 0; i < b->resLists.size(); i++) {
-        const int n = (int)b->resLists[i].size();
-        if (!n || (b->absorbed && i < b->shapes.size())) continue;   // absorbed: they run in the tiled launches
+    for (size_t i = 0; i < b->launchLists.size(); i++) {
+        const int n = (int)b->launchLists[i].size();
+        if (!n || (b->absorbed && absorbable(b, i))) continue;   // absorbed: they run in the tiled launches
         if (!forked) {
             if (!b->forkEv) HIPCHK(hipEventCreateWithFlags(&b->forkEv, hipEventDisableTiming));
             HIPCHK(hipEventRecord(b->forkEv, b->stream));
@@ -926,9 +967,14 @@ vx3h_status launchResidentAll(vx3h_batch* b, int nSteps, hipEvent_t* ev) {
         const int ns = (int)b->shapes.size();
         const int shape = (int)i % ns;
         const bool col = (int)i >= ns;
-        hipError_t e = b->realSize == 4
-            ? launchResident(b->db, rs, shape, col, b->dResLists[i], n, nSteps, evp)
-            : launchResident(*reinterpret_cast<DevBatch<double>*>(&b->db), rs, shape, col, b->dResLists[i], n, nSteps, evp);
+        const DevBatch<double>& db64 = *reinterpret_cast<DevBatch<double>*>(&b->db);
+        hipError_t e;
+        if ((int)i >= 2 * ns)
+            e = b->realSize == 4 ? launchResidentAll(b->db, rs, (int)i - 2 * ns, b->dResLists[i], n, nSteps, evp)
+                                 : launchResidentAll(db64, rs, (int)i - 2 * ns, b->dResLists[i], n, nSteps, evp);
+        else
+            e = b->realSize == 4 ? launchResident(b->db, rs, shape, col, b->dResLists[i], n, nSteps, evp)
+                                 : launchResident(db64, rs, shape, col, b->dResLists[i], n, nSteps, evp);
         if (e != hipSuccess) FAILV(VX3H_EDEVICE, std::string("resident launch failed: ") + hipGetErrorString(e));
     }
     // tiled simulations: their launch groups one after another on the tile stream
@@ -957,7 +1003,7 @@ vx3h_status launchResidentAll(vx3h_batch* b, int nSteps, hipEvent_t* ev) {
             ta.part = b->dPart;
             ta.spin = b->spinTicks;
             hipEvent_t pair[2];
-            hipEvent_t* evp = ev ? ev + 2 * (b->resLists.size() + gi) : nullptr;
+            hipEvent_t* evp = ev ? ev + 2 * (b->launchLists.size() + gi) : nullptr;
             if (!ev && b->timing) {
                 if ((st = takeEvent(b, pair[0])) || (st = takeEvent(b, pair[1]))) return st;
                 b->evUsed.push_back({pair[0], pair[1]});
@@ -1018,11 +1064,21 @@ extern "C" vx3h_status vx3h_batch_create(int device, const vx3h_batch_cfg* cfg, 
         b->shapes.assign(tmp, tmp + ns);
         // list i < ns: shape i without collisions; ns + i: shape i with collisions
         b->resLists.assign(2 * ns, {});
-        b->dResLists.assign(2 * ns, nullptr);
-        b->capRes.assign(2 * ns, 0);
-        b->resStreams.assign(2 * ns, nullptr);
-        b->joinEv.assign(2 * ns, nullptr);
-        b->joinPending.assign(2 * ns, false);
+        ResidentAllInfo all[8];
+        const DevBatch<double>& db64 = *reinterpret_cast<DevBatch<double>*>(&b->db);
+        const int na = b->realSize == 4 ? residentAllShapes(b->db, all, 8) : residentAllShapes(db64, all, 8);
+        b->allShapes.assign(all, all + na);
+        b->resPerCU.assign(ns, 1);
+        for (int i = 0; i < ns; i++)
+            if ((b->realSize == 4 ? residentOccupancy(b->db, i, &b->resPerCU[i]) : residentOccupancy(db64, i, &b->resPerCU[i])) != hipSuccess)
+                b->resPerCU[i] = 1;
+        // launch list 2 * ns + j: shape j with the links of all axes at once
+        b->launchLists.assign(2 * ns + na, {});
+        b->dResLists.assign(2 * ns + na, nullptr);
+        b->capRes.assign(2 * ns + na, 0);
+        b->resStreams.assign(2 * ns + na, nullptr);
+        b->joinEv.assign(2 * ns + na, nullptr);
+        b->joinPending.assign(2 * ns + na, false);
         // default preference: smallest voxel capacity first (more workgroups per CU), table order on ties
         for (int i = 0; i < ns; i++) b->shapePref.push_back(i);
         std::stable_sort(b->shapePref.begin(), b->shapePref.end(), [&](int x, int y) {
@@ -1045,6 +1101,7 @@ extern "C" vx3h_status vx3h_batch_create(int device, const vx3h_batch_cfg* cfg, 
         hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device);
         const hipError_t oe = b->realSize == 4 ? tiledOccupancy(b->db, b->tiledShape, &perCU)
                                                : tiledOccupancy(*reinterpret_cast<DevBatch<double>*>(&b->db), b->tiledShape, &perCU);
+        b->cus = cus;
         b->tileCap = (coop && oe == hipSuccess && khz > 0) ? perCU * cus : 0;
         b->spinTicks = (long long)khz * 1000 * 4;   // 4 s
     }
@@ -1965,16 +2022,18 @@ extern "C" vx3h_status vx3h_batch_kernel_times(vx3h_batch* b, int n_steps, doubl
     for (auto& e : ev) hipEventDestroy(e);
     // resident kernels: one launch of n_steps steps per shape in use and per tiled launch
     // group; reports the launch durations' sum
-    vx3h_status st = syncTiles(b);
+    vx3h_status st = syncResLists(b);
     if (st) return st;
-    const size_t nl = b->resLists.size() + b->tileGroups.size();
+    st = syncTiles(b);
+    if (st) return st;
+    const size_t nl = b->launchLists.size() + b->tileGroups.size();
     std::vector<hipEvent_t> rev(2 * nl, nullptr);
     for (auto& e : rev) HIPCHK(hipEventCreate(&e));
     st = launchResidentAll(b, n_steps, rev.data());
     if (st || (st = joinResident(b))) return st;
     HIPCHK(hipStreamSynchronize(b->stream));
     for (size_t i = 0; i < nl; i++) {
-        if (i < b->resLists.size() && (b->resLists[i].empty() || (b->absorbed && i < b->shapes.size()))) continue;
+        if (i < b->launchLists.size() && (b->launchLists[i].empty() || (b->absorbed && absorbable(b, i)))) continue;
         float ms = 0;
         HIPCHK(hipEventElapsedTime(&ms, rev[2 * i], rev[2 * i + 1]));
         avg_ms[5] += ms;
