@@ -14,6 +14,7 @@
 #define VX3_RES_SHAPES(X) X(512, 2, 1) X(256, 4, 2) X(256, 2, 1) X(256, 1, 1)
 // shapes with the links of all axes at once: (block, link rounds, link slots)
 #define VX3_RES_ALL_SHAPES(X) X(768, 1, 768) X(768, 2, 960)
+#define VX3_RES_ALL_TILED(X) X(768, 1, 768)
 #define VX3_RES_TABLE_FN residentShapes_f64
 #include "vx3_resident_launch.inl"
 

@@ -55,6 +55,13 @@ hipError_t launchTiled(const DevBatch<float>& b, hipStream_t s, int shape, const
                        int nSteps, hipEvent_t* ev = nullptr);
 hipError_t launchTiled(const DevBatch<double>& b, hipStream_t s, int shape, const TileArgs& ta, int nTiles, int nSync,
                        int nSteps, hipEvent_t* ev = nullptr);
+// the same with the kernel of the links of all axes at once; its shape
+hipError_t launchTiledAll(const DevBatch<float>& b, hipStream_t s, const TileArgs& ta, int nTiles, int nSync, int nSteps,
+                          hipEvent_t* ev = nullptr);
+hipError_t launchTiledAll(const DevBatch<double>& b, hipStream_t s, const TileArgs& ta, int nTiles, int nSync, int nSteps,
+                          hipEvent_t* ev = nullptr);
+hipError_t tiledAllOccupancy(const DevBatch<float>& b, ResidentAllInfo* shape, int* perCU);
+hipError_t tiledAllOccupancy(const DevBatch<double>& b, ResidentAllInfo* shape, int* perCU);
 hipError_t tiledOccupancy(const DevBatch<float>& b, int shape, int* perCU);
 hipError_t tiledOccupancy(const DevBatch<double>& b, int shape, int* perCU);
 // The fused per-step kernel over the tiles ts.tiles[0, nTiles): batch arrays into the tile

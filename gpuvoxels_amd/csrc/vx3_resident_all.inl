@@ -10,15 +10,21 @@
 // and a sign flip when reading poses and writing loads.  The sums of a voxel are taken in the
 // same order from the same values, so the results are k_resident's bit for bit.
 //
+// Tiled (TILED): the tiles of a simulation too large for one workgroup, exactly as k_resident
+// runs them (barrier, exchange records, divergence and repair launch are described there), with
+// smaller tiles.  A link between owned voxels takes a low slot, so that the wavefronts of the
+// low slots compute while the others' tiles arrive, and the links with a halo end follow.
+//
 // Included by the per-precision kernel units after vx3_resident.inl (VX_NS, real).
 
 namespace vx3 {
 namespace VX_NS {
 
-template <int BS, int LPT, int LMAX> struct ResidentAllShape {
+template <int BS, int LPT, int LMAX, bool TILED = false> struct ResidentAllShape {
     static constexpr size_t tables = VX3_RES_VMATS * sizeof(VoxMatDev) + VX3_RES_LMATS * sizeof(LinkMatDev);
     static constexpr size_t bytes = tables + (size_t)BS * (7 * sizeof(real) + 4 * sizeof(float))   // pose; thermal factor, Poisson strain
-                                  + (size_t)LMAX * (12 * sizeof(real) + 2 * sizeof(float));        // loads, end strains
+                                  + (size_t)LMAX * (12 * sizeof(real) + 2 * sizeof(float))         // loads, end strains
+                                  + (TILED ? (size_t)BS * 4 : 0);                                  // exchange voxel per slot
     static_assert(LMAX <= BS * LPT, "a slot per thread and round");
     // setup tables alias the load buffer: voxel -> slot per direction, and slot -> link
     static_assert((size_t)BS * 6 * 2 + (size_t)LMAX * 2 <= (size_t)LMAX * 12 * sizeof(real), "setup alias");
@@ -37,9 +43,9 @@ template <int BS, int LPT, int LMAX> struct ResidentAllShape {
 //   200 robots on 8^3 grids    12.3 -> 6.1     10.4 -> 5.4
 //   200 robots on 10^3 grids   13.5 -> 9.1     10.9 -> 6.8
 //   512 robots on 12^3 grids         -         22.4 -> 17.1
-template <int BS, int LPT, int LMAX>
-__global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int* simList, int nSteps) {
-    typedef ResidentAllShape<BS, LPT, LMAX> Shape;
+template <int BS, int LPT, int LMAX, bool TILED = false>
+__global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int* simList, int nSteps, TileArgs ta) {
+    typedef ResidentAllShape<BS, LPT, LMAX, TILED> Shape;
     extern __shared__ __align__(16) unsigned char smem[];
     VoxMatDev* sVM = (VoxMatDev*)smem;
     LinkMatDev* sLM = (LinkMatDev*)(smem + VX3_RES_VMATS * sizeof(VoxMatDev));
@@ -48,9 +54,11 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
     float* sTf = (float*)(sF + 12 * LMAX);
     float* sPs = sTf + BS;                      // [3][BS]
     float* sEs = sPs + 3 * BS;                  // [2][LMAX]
+    int* sXv = (int*)(sEs + 2 * LMAX);          // TILED: per slot its exchange record (as in k_resident)
     unsigned short* sVL = (unsigned short*)sF;  // [6][BS] slot of the link in direction d (setup only)
     unsigned short* sSL = sVL + 6 * BS;         // [LMAX] link of a slot (setup only)
-    __shared__ int sRun, sDiv, sExp;
+    __shared__ int sRun, sDiv;
+    __shared__ int sTile;                       // TILED: 1 = some tile diverged this step, 2 = a barrier timed out
     __shared__ double sQ[VX3_DEV_MT_MAX + 1];
     __shared__ double sRed[4][BS / 64];
     __shared__ double sCom[3], sComH0[3], sComH1[3], sAngle;   // center-of-mass history, owned by thread 0
@@ -60,10 +68,25 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
     __shared__ float sDm[VX3_RES_VMATS];        // CVX_Voxel::dampingMultiplier per voxel material (dt is fixed)
     __shared__ int sScan[BS / 64];
 
-    SimCtl& scg = b.sims[simList[blockIdx.x]];
+    TileDesc td{};
+    if (TILED) td = ta.tiles[blockIdx.x];
+    SimCtl& scg = b.sims[TILED ? td.sim : simList[blockIdx.x]];
     const int tid = threadIdx.x;
+    int divAt = -1;      // TILED: the launch's step at which a link diverged (a repair launch stops there)
+    unsigned gen = 0;    // TILED: barriers passed in this launch
     if (scg.state != 0 || (scg.flags & SC_COL_GROW)) return;
-    const int v0 = scg.v0, nv = scg.nv, l0 = scg.l0, nl = scg.nl;
+    if (TILED && ta.repair) {   // only simulations whose previous launch saw a divergence run again
+        const int dw = ta.sync[td.cOff];
+        if (!dw) return;
+        divAt = dw - 1;
+    }
+    const int v0 = scg.v0, l0 = scg.l0;
+    // the voxels this workgroup integrates, the LDS pose slots it fills, the links it computes
+    const int nv = TILED ? td.nOwn : scg.nv, nvAll = TILED ? td.nOwn + td.nHalo : scg.nv, nl = TILED ? td.nLinks : scg.nl;
+    auto gvox = [&](int slot) { return v0 + (TILED ? ta.vox[td.vOff + slot] & 0x7fffffff : slot); };
+    auto glink = [&](int j) { return l0 + (TILED ? ta.link[td.lOff + j] & 0x7fffffff : j); };
+    // vneg | vpos << 16, as slots
+    auto endsOf = [&](int l) { return TILED ? ta.ends[td.lOff + l] : (b.lneg[l0 + l] - v0) | ((b.lpos[l0 + l] - v0) << 16); };
     const double dt = scg.dt;
     const float dtf = scg.dt;
     const real nom = (real)scg.voxSize;
@@ -82,32 +105,37 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
     for (int i = 0; i < nlm; i++)
         ldsCopyWords((int*)&sLM[i], (const int*)&b.lmatTab[b.simMats[mat0 + nvm + i]], sizeof(LinkMatDev) / 4, tid, BS);
     for (int i = tid; i < 6 * BS; i += BS) sVL[i] = 0xFFFF;
-    // links that took the expensive branches last step in the lowest slots, the others after
-    // them, each in link order (see k_resident)
-    auto expensive = [&](int g) {
+    // the lowest slots: the links that took the expensive branches last step (see k_resident);
+    // TILED, those between owned voxels, which do not wait for the other tiles.  The others after
+    // them, each in link order.
+    auto early = [&](int l) {
+        if (TILED) {
+            const int e = endsOf(l);
+            return (e & 0xFFFF) < nv && (e >> 16) < nv;
+        }
+        const int g = l0 + l;
         const real x = b.a2x[g], y = b.a2y[g], z = b.a2z[g];
         return !(b.lflags[g] & LF_SMALL_ANGLE) || x * x + y * y + z * z > (real)0.009;
     };
-    int nExp = 0;
+    int mine = 0;
 #pragma unroll
     for (int k = 0; k < LPT; k++) {
         const int l = tid * LPT + k;
-        if (l < nl && expensive(l0 + l)) nExp++;
+        if (l < nl && early(l)) mine++;
     }
-    int allExp;
-    int exAt = resBlockScan<BS>(nExp, sScan, &allExp);
+    int nEarly;
+    int at = resBlockScan<BS>(mine, sScan, &nEarly);
 #pragma unroll
     for (int k = 0; k < LPT; k++) {   // thread tid places links [tid * LPT, tid * LPT + LPT)
         const int l = tid * LPT + k;
         if (l >= nl) continue;
-        const int g = l0 + l;
-        const bool ex = expensive(g);
-        const int slot = ex ? exAt : allExp + l - exAt;   // exAt: the expensive ones before l
-        exAt += ex;
-        const int ax = b.lmeta[g] & 3;
+        const bool first = early(l);
+        const int slot = first ? at : nEarly + l - at;   // at: the early ones before l
+        at += first;
+        const int ax = b.lmeta[glink(l)] & 3, e = endsOf(l);
         sSL[slot] = (unsigned short)l;
-        sVL[(2 * ax) * BS + b.lneg[g] - v0] = (unsigned short)slot;
-        sVL[(2 * ax + 1) * BS + b.lpos[g] - v0] = (unsigned short)slot;
+        sVL[(2 * ax) * BS + (e & 0xFFFF)] = (unsigned short)slot;
+        sVL[(2 * ax + 1) * BS + (e >> 16)] = (unsigned short)slot;
     }
     // 2*sqrt(m)*zeta/previousDt (VX_Voxel.h:131): the first step's previousDt is the dt of the
     // simulation's last step (which a caller-given dt may have set), every later one the launch's dt
@@ -133,9 +161,9 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
         const int slot = tid + k * BS;
         lEnds[k] = -1;
         if (slot >= nl) continue;
-        const int l = sSL[slot], g = l0 + l;
+        const int l = sSL[slot], g = glink(l);
         lIdx[k] = l;
-        lEnds[k] = (b.lneg[g] - v0) | ((b.lpos[g] - v0) << 16);
+        lEnds[k] = endsOf(l);
         lMats[k] = localLmat(b.lmeta[g] >> 2) | (localVmat(b.vmat[b.lneg[g]]) << 8) | (localVmat(b.vmat[b.lpos[g]]) << 16) |
                    ((b.lmeta[g] & 3) << 24);
         ls[k].pos2 = V3<real>(b.q2x[g], b.q2y[g], b.q2z[g]);
@@ -157,7 +185,7 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
         bool over = false;
         for (int base = 0; base < nv && !over; base += 64) {
             const int v = base + tid;
-            const long long ph = v < nv ? __double_as_longlong(b.phase[v0 + v]) : 0;
+            const long long ph = v < nv ? __double_as_longlong(b.phase[gvox(v)]) : 0;
             bool pending = v < nv;
             while (!over && __any(pending)) {
                 const int src = __ffsll((unsigned long long)__ballot(pending)) - 1;   // lowest pending lane
@@ -187,7 +215,7 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
     int vl[3] = {-1, -1, -1};   // slots of directions (2i, 2i+1) packed lo | hi << 16, 0xFFFF = none
     int vpm = 0;                // CVX_Voxel::strain's per-axis case, fixed for the launch (see k_resident)
     if (tid < nv) {
-        const int g = v0 + tid;
+        const int g = gvox(tid);
         vm = V3<real>(b.mx[g], b.my[g], b.mz[g]);
         va = V3<real>(b.ax[g], b.ay[g], b.az[g]);
         vf = b.vflags[g];
@@ -204,6 +232,10 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
             const bool tension = (n == 2) || (ext && n == 1 && ((ext->dofFixed & (1 << i)) || ext->force[i] != 0));
             vpm |= (n == 2 ? 1 << i : 0) | (tension ? 8 << i : 0);
         }
+    }
+    if (TILED) sXv[tid] = tid < nvAll ? ta.xidx[td.vOff + tid] : -1;
+    if (tid < nvAll) {
+        const int g = gvox(tid);
         const real* src[7] = {b.px, b.py, b.pz, b.ow, b.ox, b.oy, b.oz};
 #pragma unroll
         for (int q = 0; q < 7; q++) sP[q * BS + tid] = src[q][g];
@@ -214,9 +246,9 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
 #pragma unroll
         for (int k = 0; k < LPT; k++) {
             if (lEnds[k] < 0) continue;
-            const int slot = tid + k * BS, ax = lMats[k] >> 24;
-            sEs[slot] = b.es[(2 * ax) * VC + v0 + (lEnds[k] & 0xFFFF)];
-            sEs[LMAX + slot] = b.es[(2 * ax + 1) * VC + v0 + (lEnds[k] >> 16)];
+            const int slot = tid + k * BS, ax = lMats[k] >> 24, g = glink(lIdx[k]);
+            sEs[slot] = b.es[(2 * ax) * VC + b.lneg[g]];
+            sEs[LMAX + slot] = b.es[(2 * ax + 1) * VC + b.lpos[g]];
         }
     }
     double t = scg.t;
@@ -229,6 +261,58 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
         sAngle = scg.recentAngle;
     }
     __syncthreads();   // setup tables alias the load buffer: done with them
+    // TILED: the second half of the simulation's barrier `gen`, whose arrival is pending:
+    // wait for every tile, then (sampleNow) the tiles' centre-of-mass partial sums in tile
+    // order into sRed[.][0], then (loadHalo) the halo poses into LDS.  1: some tile saw a
+    // link diverge (leave; the repair launch takes over), 2: a tile did not arrive (the
+    // simulation fails).
+    bool pend = false;
+    auto finishBarrier = [&](bool loadHalo, bool sampleNow) -> int {
+        if (tid < 64) {   // the first wave; tile 0 of the simulation is workgroup blockIdx.x - td.tile
+            int flag = 0;
+            if (!tileWait(ta.sync + ta.flag0 + (blockIdx.x - td.tile), td.nTiles, gen, ta.repair, ta.spin)) flag = 2;
+            else if (divAt < 0 && xget(ta.sync + td.cOff)) flag = 1;
+            if (tid == 0) sTile = flag;
+        }
+        const int par = gen & 1;
+        gen++;
+        pend = false;
+        __syncthreads();
+        if (sTile == 2) {   // state stays as it was
+            if (tid == 0) scg.state = 4;
+            return 2;
+        }
+        if (sTile == 1) return 1;   // state untouched: the repair launch runs it to that step's link pass
+        if (sampleNow) {   // the partial sums read in parallel, added in tile order by one thread
+            const double* P = ta.part + td.pOff + (size_t)par * td.nTiles * 4;
+            double* sP = (double*)sF;   // the load buffer is free between the voxel and link passes
+            for (int j = tid; j < td.nTiles; j += BS) {
+                const double a0 = xget(P + 4 * j), a1 = xget(P + 4 * j + 1), a2 = xget(P + 4 * j + 2), a3 = xget(P + 4 * j + 3);
+                sP[4 * j] = a0; sP[4 * j + 1] = a1; sP[4 * j + 2] = a2; sP[4 * j + 3] = a3;
+            }
+            __syncthreads();
+            if (tid == 0) {   // the same totals in every tile
+                for (int q = 0; q < 4; q++) sRed[q][0] = 0;
+                for (int j = 0; j < td.nTiles; j++)
+                    for (int q = 0; q < 4; q++) sRed[q][0] += sP[4 * j + q];
+            }
+        }
+        if (loadHalo) {
+            const real* X = (const real*)ta.xch + td.xOff + (size_t)par * td.xPar;
+            if (tid >= nv && tid < nvAll) {
+                // every load issued before the first LDS write: one memory latency, not eleven
+                const real* r = X + (size_t)sXv[tid] * VX3_XCH_STRIDE;
+                real q[VX3_XCH_STRIDE - 1];
+#pragma unroll
+                for (int f = 0; f < VX3_XCH_STRIDE - 1; f++) q[f] = xget(r + f);
+#pragma unroll
+                for (int f = 0; f < 7; f++) sP[f * BS + tid] = q[f];
+                sTf[tid] = (float)q[7]; sPs[tid] = (float)q[8]; sPs[BS + tid] = (float)q[9]; sPs[2 * BS + tid] = (float)q[10];
+            }
+            __syncthreads();
+        }
+        return 0;
+    };
     for (int it = 0; it < nSteps; it++) {
         // keep per-step LDS address arithmetic inside the loop (register pressure)
 #pragma unroll
@@ -237,14 +321,12 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
         // temperatures of this step's distinct phases (read in the voxel pass, after the link barrier)
         if (vary && tid < nph) sPhT[tid] = actuationTemp(tempAmp, tempPeriod, sPhase[tid], t + dt, expansion);
         // ---- links
-#pragma unroll
-        for (int k = 0; k < LPT; k++) {
-            if (lEnds[k] < 0) continue;
+        auto linkAt = [&](int k) {
             const int slot = tid + k * BS, vn = lEnds[k] & 0xFFFF, vq = lEnds[k] >> 16, a = lMats[k] >> 24;
             const LinkMatDev& mat = sLM[lMats[k] & 0xFF];
             const int in_ = (lMats[k] >> 8) & 0xFF, ip_ = (lMats[k] >> 16) & 0xFF;
             const VoxMatDev &mn = sVM[in_], &mp = sVM[ip_];
-            if (mn.fixed && mp.fixed) continue;   // its slots are never read: both ends are fixed
+            if (mn.fixed && mp.fixed) return;   // its slots are never read: both ends are fixed
             const int cy = a == 1 ? 0 : 1, cz = a == 2 ? 0 : 2;   // components read as the frame's y and z (x: a)
             const real restLength = (real)0.5 * (nom * (real)sTf[vn] + nom * (real)sTf[vq]);
             float area, tss;
@@ -289,10 +371,26 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
                 sEs[LMAX + slot] = 2.0f * ls[k].strain * r / (1.0f + r);
             }
             if (ls[k].strain > 100) sDiv = 1;
+        };
+        if (TILED && pend) {
+            // those between owned voxels, then the wait and the halo, then those with a halo end
+#pragma unroll
+            for (int k = 0; k < LPT; k++)
+                if (tid + k * BS < nEarly) linkAt(k);
+            if (finishBarrier(true, false)) return;
+#pragma unroll
+            for (int k = 0; k < LPT; k++)
+                if (lEnds[k] >= 0 && tid + k * BS >= nEarly) linkAt(k);
+        } else {
+#pragma unroll
+            for (int k = 0; k < LPT; k++)
+                if (lEnds[k] >= 0) linkAt(k);
         }
         __syncthreads();
         // ---- voxels
-        const bool diverged = sDiv != 0;
+        // (a tile learns of its simulation's divergence only at the step's barrier and stops at that
+        // step on a second run)
+        const bool diverged = TILED ? it == divAt : sDiv != 0;
         steps++;
         const bool sample = !diverged && cycleStep > 0 && steps % cycleStep == 0;
         double psx = 0, psy = 0, psz = 0, psm = 0;
@@ -341,6 +439,13 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
                 psx = (double)vp.x * mass; psy = (double)vp.y * mass; psz = (double)vp.z * mass;
                 psm = mass;
             }
+            if (TILED && sXv[tid] >= 0) {   // a voxel another tile reads: its record out as soon as it is final
+                real q[VX3_XCH_STRIDE - 1] = {sP[tid], sP[BS + tid], sP[2 * BS + tid], sP[3 * BS + tid], sP[4 * BS + tid], sP[5 * BS + tid],
+                                              sP[6 * BS + tid], (real)sTf[tid], (real)sPs[tid], (real)sPs[BS + tid], (real)sPs[2 * BS + tid]};
+                real* r = (real*)ta.xch + td.xOff + (size_t)(gen & 1) * td.xPar + (size_t)sXv[tid] * VX3_XCH_STRIDE;
+#pragma unroll
+                for (int f = 0; f < VX3_XCH_STRIDE - 1; f++) xput(r + f, q[f]);
+            }
         }
         if (sample) {
             // FP64 center of mass of the measured voxels (VX3_VoxelyzeKernel.cu:477-493)
@@ -350,13 +455,36 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
             }
             if ((tid & 63) == 0) { sRed[0][tid >> 6] = psx; sRed[1][tid >> 6] = psy; sRed[2][tid >> 6] = psz; sRed[3][tid >> 6] = psm; }
         }
-        if (sample) {
+        if (TILED && !diverged) {
+            // ---- arrival at the simulation's barrier (TILED): the records are out; the wait
+            // comes in the next step's link pass, or now on a sampling step (the centre of
+            // mass needs every tile's partial sum)
+            __builtin_amdgcn_s_waitcnt(0);   // this thread's exchange stores are complete
             __syncthreads();
+            if (tid == 0) {
+                if (sample) {
+                    double* P = ta.part + td.pOff + (size_t)(gen & 1) * td.nTiles * 4;
+                    double tot[4] = {0, 0, 0, 0};
+                    for (int w = 0; w < BS / 64; w++)
+                        for (int q = 0; q < 4; q++) tot[q] += sRed[q][w];
+                    for (int q = 0; q < 4; q++) xput(P + 4 * td.tile + q, tot[q]);
+                }
+                if (sDiv) __hip_atomic_fetch_max(ta.sync + td.cOff, it + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                tileArrive(ta.sync + ta.flag0 + blockIdx.x, gen, ta.repair);
+            }
+            pend = true;
+            if (sample && finishBarrier(true, true)) return;
+        } else if (sample) __syncthreads();
+        if (sample) {
             angleSamples++;
             if (tid == 0) {
                 double tot[4] = {0, 0, 0, 0};
-                for (int w = 0; w < BS / 64; w++)
-                    for (int q = 0; q < 4; q++) tot[q] += sRed[q][w];
+                if (TILED) {
+                    for (int q = 0; q < 4; q++) tot[q] = sRed[q][0];
+                } else {
+                    for (int w = 0; w < BS / 64; w++)
+                        for (int q = 0; q < 4; q++) tot[q] += sRed[q][w];
+                }
                 double* A = sComH0; double* B = sComH1; double* C = sCom;
                 for (int q = 0; q < 3; q++) { A[q] = B[q]; B[q] = C[q]; C[q] = tot[3] == 0 ? 0.0 : (1.0 / tot[3]) * tot[q]; }
                 const bool bc = B[0] == C[0] && B[1] == C[1] && B[2] == C[2];
@@ -375,17 +503,23 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
         if (diverged) { state = 2; break; }
         t = tn;
         bool stop = maxSteps > 0 && steps >= maxSteps;
-        if (!stop && stopLen > 0 && tid == 0) sRun = mathTreeEval(b.tokens + stopOff, stopLen, sCom[0], sCom[1], sCom[2], 0, t, sAngle, 0, 0, nv, sQ) > 0 ? 0 : 1;
+        if (!stop && stopLen > 0 && tid == 0) sRun = mathTreeEval(b.tokens + stopOff, stopLen, sCom[0], sCom[1], sCom[2], 0, t, sAngle, 0, 0, scg.nv, sQ) > 0 ? 0 : 1;
         if (it == 0 && prevDt0 != dtf && tid < nvm) sDm[tid] = 2 * sVM[tid].sqrtMass * sVM[tid].zetaInternal / (sVM[tid].fixed ? 0.0f : dtf);
         __syncthreads();   // next step's link pass reads the new poses
-        if (stop || !sRun) { state = 1; break; }
+        if (stop || !sRun) {
+            if (TILED && pend && finishBarrier(false, false)) return;
+            state = 1;
+            break;
+        }
     }
+    if (TILED && pend && finishBarrier(false, false)) return;   // the launch's last step
 
     // ---- write back in the stream layout
 #pragma unroll
     for (int k = 0; k < LPT; k++) {
         if (lEnds[k] < 0) continue;
-        const int g = l0 + lIdx[k];
+        if (TILED && !(ta.link[td.lOff + lIdx[k]] & 0x80000000)) continue;   // the other tile writes it
+        const int g = glink(lIdx[k]);
         b.q2x[g] = ls[k].pos2.x; b.q2y[g] = ls[k].pos2.y; b.q2z[g] = ls[k].pos2.z;
         b.a1x[g] = ls[k].a1v.x; b.a1y[g] = ls[k].a1v.y; b.a1z[g] = ls[k].a1v.z;
         b.a2x[g] = ls[k].a2v.x; b.a2y[g] = ls[k].a2v.y; b.a2z[g] = ls[k].a2v.z;
@@ -395,12 +529,12 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
         b.lflags[g] = ls[k].flags;
         if (poisson) {
             const int slot = tid + k * BS, ax = lMats[k] >> 24;
-            b.es[(2 * ax) * VC + v0 + (lEnds[k] & 0xFFFF)] = sEs[slot];
-            b.es[(2 * ax + 1) * VC + v0 + (lEnds[k] >> 16)] = sEs[LMAX + slot];
+            b.es[(2 * ax) * VC + b.lneg[g]] = sEs[slot];
+            b.es[(2 * ax + 1) * VC + b.lpos[g]] = sEs[LMAX + slot];
         }
     }
     if (tid < nv) {
-        const int g = v0 + tid;
+        const int g = gvox(tid);
         real* dst[7] = {b.px, b.py, b.pz, b.ow, b.ox, b.oy, b.oz};
 #pragma unroll
         for (int q = 0; q < 7; q++) dst[q][g] = sP[q * BS + tid];
@@ -410,7 +544,7 @@ __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int
         b.tfac[g] = sTf[tid];
         b.psx[g] = sPs[tid]; b.psy[g] = sPs[BS + tid]; b.psz[g] = sPs[2 * BS + tid];
     }
-    if (tid == 0) {
+    if (tid == 0 && (!TILED || td.tile == 0)) {   // every tile holds the same control values
         if (steps != scg.steps) scg.prevDt = dtf;
         scg.t = t;
         scg.steps = steps;

@@ -111,7 +111,10 @@ struct SlotHost {
     int nlSeen = 0;              // links known to the host shadows below (nl + attached ones read back)
     int shape = -1;              // resident kernel shape, -1 = stream path (or tiled)
     int tiles = 0;               // > 0: runs on the tiled resident kernel as this many workgroups
-    TilePlan tplan;              // its tiles (sim-local; the tables themselves live on the device)
+    TilePlan tplan, fplan;       // its tiles (sim-local): for the axis-by-axis kernel, and finer ones (planned when first
+                                 // used) for the kernel with the links of all axes at once
+    bool fine = false;           // the device tables are the finer ones'
+    int fineSlots = 0;           // owned and halo voxels of a tile that fplan was planned for (0: not yet)
     int tv0 = 0, tvN = 0, tl0 = 0, tlN = 0, tx0 = 0, txN = 0, tp0 = 0;   // its ranges in the tile pools
     bool oneTile = false;        // a one-workgroup simulation with one-tile tables in the pools
     int axisLinks = 0;           // links on its busiest axis
@@ -208,6 +211,9 @@ struct vx3h_batch {
     // one after another on tileStream beside the other paths
     int tiledShape = -1;                         // shape of the tiled kernel: the largest voxel capacity
     int tileCap = 0;                             // workgroups of it the device holds at once (0: no tiling)
+    ResidentAllInfo fineShape{0, 0};             // the same for the finer tiles
+    int fineCap = 0;
+    bool fine = false;                           // the launch groups are of finer tiles
     long long spinTicks = 0;                     // a tile's longest barrier wait, in wall-clock ticks
     std::vector<int> tiledSims;                  // slots, in admission order
     bool tileDirty = false;
@@ -676,6 +682,90 @@ vx3h_status ensureOneTile(vx3h_batch* b, int s) {
     return VX3H_OK;
 }
 
+// Puts a simulation's tile tables into the pools.
+vx3h_status placeTiles(vx3h_batch* b, SlotHost& sh, const TilePlan& p) {
+    vx3h_status st;
+    sh.tvN = (int)p.vox.size();
+    sh.tlN = std::max(1, (int)p.link.size());
+    sh.txN = std::max(1, p.nPub);
+    sh.tiles = (int)p.tiles.size();
+    if ((st = poolAlloc(b, b->tileSlotPool, sh.tvN, sh.tv0)) || (st = poolAlloc(b, b->tileLinkPool, sh.tlN, sh.tl0)) ||
+        (st = poolAlloc(b, b->tileXchPool, sh.txN, sh.tx0)) || (st = poolAlloc(b, b->tilePartPool, sh.tiles, sh.tp0)))
+        return st;
+    if ((st = upload(b, b->dTileVox + sh.tv0, p.vox.data(), p.vox.size() * 4)) ||
+        (st = upload(b, b->dTileXidx + sh.tv0, p.xidx.data(), p.xidx.size() * 4)) ||
+        (st = upload(b, b->dTileLink + sh.tl0, p.link.data(), p.link.size() * 4)) ||
+        (st = upload(b, b->dTileEnds + sh.tl0, p.ends.data(), p.ends.size() * 4)))
+        return st;
+    return VX3H_OK;
+}
+
+void releaseTiles(vx3h_batch* b, SlotHost& sh) {
+    b->tileSlotPool.ra.release(sh.tv0, sh.tvN);
+    b->tileLinkPool.ra.release(sh.tl0, sh.tlN);
+    b->tileXchPool.ra.release(sh.tx0, sh.txN);
+    b->tilePartPool.ra.release(sh.tp0, sh.tiles);
+}
+
+// Whether the tiled simulations step as finer tiles on the kernel with the links of all axes at
+// once, and their plans and tables for it.  Its step takes about half as long, but its tiles are
+// smaller (the loads of all their links share LDS), so that is done while one launch holds all
+// of them and nothing else shares the chip; else fewer, larger tiles get more done.  Plans of
+// 448 slots a tile where these fit too (2.6 times the tiles), else as large as the shape takes
+// (1.6 to 2.1 times): still smaller ones wait for as many more barriers as they save.  Measured
+// on MI355X, us per step, the shape's own size -> 448 slots; axis by axis in brackets:
+//                                        FP32                     FP64
+//   one robot on a 14^3 grid       9.2 -> 9.0 (13.8)       12.0 -> 10.8 (19.8)
+//   three on 30^3                 10.6 -> 10.1 (15.9)      13.6 -> 12.3 (23.9)
+//   one on 45^3                   11.2 -> 10.2 (16.3)      13.8 -> 12.5 (24.5)
+// 320 slots: 9.1, 9.7, 10.2 and 11.0, 11.7, 12.1.
+vx3h_status chooseTiles(vx3h_batch* b) {
+    bool fine = b->fineCap > 1 && b->cfg.block_size == 0 && !b->tiledSims.empty() && !b->nStreamSims && b->stepSims.empty();
+    for (const auto& L : b->resLists) fine = fine && L.empty();
+    const size_t cap = b->fineCap;
+    size_t coarse = 0, tiles = 0;
+    for (int s : b->tiledSims) coarse += b->slots[s].tplan.tiles.size();
+    fine = fine && 3 * coarse <= 2 * cap;
+    const int slots = std::min(5 * coarse <= 2 * cap ? 448 : INT32_MAX, b->fineShape.block);
+    for (size_t i = 0; fine && i < b->tiledSims.size(); i++) {
+        SlotHost& sh = b->slots[b->tiledSims[i]];
+        if (sh.fineSlots != slots) {
+            std::vector<int> axis(sh.nl);
+            for (int v = 0; v < sh.nv; v++)
+                for (int a = 0; a < 3; a++) {
+                    const int l = sh.vlinks[6 * (size_t)v + 2 * a];
+                    if (l >= 0) axis[l] = a;
+                }
+            TilePlan p;
+            if (!planTiles(sh.nv, sh.ijk.data(), sh.nl, sh.lneg.data(), sh.lpos.data(), axis.data(), slots, b->fineShape.links / 3,
+                           b->fineCap, &p, false))
+                p = TilePlan();
+            if (sh.fine) {   // its tables are the old plan's
+                HIPCHK(hipStreamSynchronize(b->stream));
+                releaseTiles(b, sh);
+                sh.fine = false;
+                if (vx3h_status st = placeTiles(b, sh, sh.tplan)) return st;
+            }
+            sh.fplan = std::move(p);
+            sh.fineSlots = slots;
+        }
+        tiles += sh.fplan.tiles.size();
+        fine = sh.fplan.tiles.size() > 1 && tiles <= cap;
+    }
+    b->fine = fine;
+    bool synced = false;
+    for (int s : b->tiledSims) {
+        SlotHost& sh = b->slots[s];
+        if (sh.fine == fine) continue;
+        if (!synced) HIPCHK(hipStreamSynchronize(b->stream));   // launches that read the tables
+        synced = true;
+        releaseTiles(b, sh);
+        sh.fine = fine;
+        if (vx3h_status st = placeTiles(b, sh, fine ? sh.fplan : sh.tplan)) return st;
+    }
+    return VX3H_OK;
+}
+
 // The tiled launch groups, after a simulation joined or left: whole simulations packed
 // into groups of at most tileCap tiles (first fit, largest first: a launch lasts as long
 // per step whether full or not), and their tile descriptors pointing at each
@@ -683,6 +773,8 @@ vx3h_status ensureOneTile(vx3h_batch* b, int s) {
 // holds one divergence word per simulation, then one arrival flag per workgroup.
 vx3h_status syncTiles(vx3h_batch* b) {
     if (!b->tileDirty) return VX3H_OK;
+    vx3h_status fs = chooseTiles(b);
+    if (fs) return fs;
     std::vector<int> order = b->tiledSims;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->slots[x].tiles > b->slots[y].tiles; });
     // with tiled simulations running, the one-workgroup simulations without collisions
@@ -705,7 +797,7 @@ vx3h_status syncTiles(vx3h_batch* b) {
     std::vector<int> fill;
     for (int s : order) {
         size_t i = 0;
-        while (i < bins.size() && fill[i] + tilesOf(s) > b->tileCap) i++;
+        while (i < bins.size() && fill[i] + tilesOf(s) > (b->fine ? b->fineCap : b->tileCap)) i++;
         if (i == bins.size()) { bins.emplace_back(); fill.push_back(0); }
         bins[i].push_back(s);
         fill[i] += tilesOf(s);
@@ -717,12 +809,13 @@ vx3h_status syncTiles(vx3h_batch* b) {
         vx3h_batch::TileGroup g{(int)T.size(), 0, syncTot, 0};
         for (int s : bin) {
             const SlotHost& sh = b->slots[s];
-            for (TileDesc d : sh.tplan.tiles) {
+            const TilePlan& plan = sh.fine ? sh.fplan : sh.tplan;
+            for (TileDesc d : plan.tiles) {
                 d.sim = s;
                 d.vOff += sh.tv0;
                 d.lOff += sh.tl0;
                 d.xOff = sh.tx0 * 2 * VX3_XCH_STRIDE;
-                d.xPar = VX3_XCH_STRIDE * sh.tplan.nPub;
+                d.xPar = VX3_XCH_STRIDE * plan.nPub;
                 d.cOff = g.nSync;
                 d.pOff = sh.tp0 * 8;
                 T.push_back(d);
@@ -1010,7 +1103,11 @@ vx3h_status launchResidentAll(vx3h_batch* b, int nSteps, hipEvent_t* ev) {
                 b->timedSteps += nSteps;
                 evp = pair;
             }
-            const hipError_t e = b->realSize == 4
+            const hipError_t e = b->fine
+                ? (b->realSize == 4 ? launchTiledAll(b->db, b->tileStream, ta, g.count, g.nSync + g.count, nSteps, evp)
+                                    : launchTiledAll(*reinterpret_cast<DevBatch<double>*>(&b->db), b->tileStream, ta, g.count,
+                                                     g.nSync + g.count, nSteps, evp))
+                : b->realSize == 4
                 ? launchTiled(b->db, b->tileStream, b->tiledShape, ta, g.count, g.nSync + g.count, nSteps, evp)
                 : launchTiled(*reinterpret_cast<DevBatch<double>*>(&b->db), b->tileStream, b->tiledShape, ta, g.count,
                               g.nSync + g.count, nSteps, evp);
@@ -1104,6 +1201,10 @@ extern "C" vx3h_status vx3h_batch_create(int device, const vx3h_batch_cfg* cfg, 
         b->cus = cus;
         b->tileCap = (coop && oe == hipSuccess && khz > 0) ? perCU * cus : 0;
         b->spinTicks = (long long)khz * 1000 * 4;   // 4 s
+        int finePerCU = 0;
+        const hipError_t fe = b->realSize == 4 ? tiledAllOccupancy(b->db, &b->fineShape, &finePerCU)
+                                               : tiledAllOccupancy(db64, &b->fineShape, &finePerCU);
+        b->fineCap = (coop && fe == hipSuccess && khz > 0) ? finePerCU * cus : 0;
     }
     size_t freeB = 0, totB = 0;
     if (hipMemGetInfo(&freeB, &totB) != hipSuccess) freeB = 0;
@@ -1687,23 +1788,9 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     sh.nb0 = nb0; sh.nbN = nbN; sh.h0 = h0; sh.hN = hN; sh.near0 = near0; sh.nearN = nearN; sh.c0 = c0;
     sh.tg0 = tg0; sh.nTg = nTg;
     sh.at0 = at0; sh.ap0 = ap0; sh.apN = apN;
-    if (tiles) {   // the tile tables into their pools, once
-        vx3h_status st;
-        sh.tvN = (int)tplan.vox.size();
-        sh.tlN = std::max(1, (int)tplan.link.size());
-        sh.txN = std::max(1, tplan.nPub);
-        if ((st = poolAlloc(b, b->tileSlotPool, sh.tvN, sh.tv0)) || (st = poolAlloc(b, b->tileLinkPool, sh.tlN, sh.tl0)) ||
-            (st = poolAlloc(b, b->tileXchPool, sh.txN, sh.tx0)) || (st = poolAlloc(b, b->tilePartPool, tiles, sh.tp0)))
-            return st;
-        UPLOAD(b->dTileVox + sh.tv0, tplan.vox.data(), tplan.vox.size() * 4);
-        UPLOAD(b->dTileXidx + sh.tv0, tplan.xidx.data(), tplan.xidx.size() * 4);
-        if (!tplan.link.empty()) {
-            UPLOAD(b->dTileLink + sh.tl0, tplan.link.data(), tplan.link.size() * 4);
-            UPLOAD(b->dTileEnds + sh.tl0, tplan.ends.data(), tplan.ends.size() * 4);
-        }
-        sh.tiles = tiles;
-        sh.tplan.tiles = std::move(tplan.tiles);   // the descriptors stay on the host
-        sh.tplan.nPub = tplan.nPub;
+    if (tiles) {
+        sh.tplan = std::move(tplan);
+        if (vx3h_status st = placeTiles(b, sh, sh.tplan)) return st;
         b->tiledSims.push_back(s);
         b->tileDirty = true;
     } else if (shape >= 0) {   // the kernel variant with contacts for a simulation with collisions
@@ -1717,6 +1804,7 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
         b->stepDirty = true;
     }
     else b->nStreamSims++;
+    if (!tiles && shape < 0) b->tileDirty = true;   // which tiles run depends on what else does
     sh.vlinks = H.voxelLinks;
     sh.surface.resize(NV);
     for (int i = 0; i < NV; i++) sh.surface[i] = (H.vflags[i] & VF_INTERIOR) ? 0 : 1;
@@ -2392,10 +2480,7 @@ extern "C" vx3h_status vx3h_sim_retire(vx3h_batch* b, int slot) {
     }
     if (sh.tiles) {
         b->tiledSims.erase(std::remove(b->tiledSims.begin(), b->tiledSims.end(), slot), b->tiledSims.end());
-        b->tileSlotPool.ra.release(sh.tv0, sh.tvN);
-        b->tileLinkPool.ra.release(sh.tl0, sh.tlN);
-        b->tileXchPool.ra.release(sh.tx0, sh.txN);
-        b->tilePartPool.ra.release(sh.tp0, sh.tiles);
+        releaseTiles(b, sh);
         b->tileDirty = true;
     } else if (sh.shape >= 0) {
         auto& L = b->resLists[sh.shape];
@@ -2405,8 +2490,8 @@ extern "C" vx3h_status vx3h_sim_retire(vx3h_batch* b, int slot) {
     } else if (!sh.stepTiles.empty()) {
         b->stepSims.erase(std::remove(b->stepSims.begin(), b->stepSims.end(), slot), b->stepSims.end());
         releaseStep(b, sh);
-        b->stepDirty = true;
-    } else b->nStreamSims--;
+        b->stepDirty = b->tileDirty = true;
+    } else { b->nStreamSims--; b->tileDirty = true; }
     if (sh.oneTile) {
         b->tileSlotPool.ra.release(sh.tv0, sh.tvN);
         b->tileLinkPool.ra.release(sh.tl0, sh.tlN);

@@ -18,7 +18,7 @@ struct Planner {
     const int *ijk = nullptr, *lneg = nullptr, *lpos = nullptr, *laxis = nullptr;
     int vmax = 0, lax = 0;
     std::vector<int> inc0, inc;   // links incident to each voxel (CSR)
-    std::vector<int> vmark, lmark;
+    std::vector<int> vmark, lmark, count, aside;
     int epoch = 0;
     bool failed = false;
     std::vector<std::vector<int>> parts;
@@ -56,7 +56,8 @@ struct Planner {
                 if (vmark[u] != own && vmark[u] != halo) { vmark[u] = halo; nh++; }
             }
         }
-        lastNeed = (int)n + nh;
+        // (links past lax: as many slots too many)
+        lastNeed = std::max((int)n + nh, (int)((long long)std::max(per[0], std::max(per[1], per[2])) * vmax / lax));
         return (int)n + nh <= vmax && per[0] <= lax && per[1] <= lax && per[2] <= lax;
     }
 
@@ -82,11 +83,25 @@ struct Planner {
         const int kl = k / 2;
         size_t m = (size_t)((double)n * kl / k + 0.5);
         m = std::max<size_t>(1, std::min(m, n - 1));
-        // the m lowest along the axis (ties by voxel index): a selection, not a sort
-        std::nth_element(part, part + m, part + n, [&](int x, int y) {
-            const int cx = ijk[3 * x + ax], cy = ijk[3 * y + ax];
-            return cx != cy ? cx < cy : x < y;
-        });
+        // the m lowest along the axis, ties in the order they come (by voxel index): a histogram of
+        // the coordinate finds the cut, so a level costs two passes and keeps the order
+        count.assign(hi[ax] - lo[ax] + 1, 0);
+        for (size_t i = 0; i < n; i++) count[ijk[3 * part[i] + ax] - lo[ax]]++;
+        int at = 0;
+        size_t below = 0;
+        while (below + count[at] < m) below += count[at++];
+        size_t ties = m - below, j = 0, r = 0;
+        at += lo[ax];
+        aside.resize(std::max(aside.size(), n));
+        for (size_t i = 0; i < n; i++) {
+            const int v = part[i], c = ijk[3 * v + ax];
+            if (c < at || (c == at && ties > 0)) {
+                if (c == at) ties--;
+                part[j++] = v;
+            } else
+                aside[r++] = v;
+        }
+        std::copy(aside.begin(), aside.begin() + r, part + j);
         cut(part, m, kl);
         cut(part + m, n - m, k - kl);
     }
@@ -95,7 +110,7 @@ struct Planner {
 }  // namespace
 
 bool planTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos, const int* laxis, int vmax, int lax,
-               int maxTiles, TilePlan* out) {
+               int maxTiles, TilePlan* out, bool fewest) {
     if (nv <= 0 || vmax <= 0 || lax <= 0 || maxTiles <= 0 || vmax > 0xFFFF) return false;
     Planner p;
     p.nv = nv; p.nl = nl; p.ijk = ijk; p.lneg = lneg; p.lpos = lpos; p.laxis = laxis; p.vmax = vmax; p.lax = lax;
@@ -105,7 +120,7 @@ bool planTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos,
     // size that all fit.  From the count at which the blocks would fill every slot, a plan
     // that fails tries next the count at which its overflowing block's owned + halo would
     // have fit (blocks of n voxels need about n (1 + halo ratio) slots); the first count
-    // that fits is then lowered one at a time towards the last that failed.  A shape no
+    // that fits is then (fewest) lowered one at a time towards the last that failed.  A shape no
     // equal split fits falls back to halving the blocks that do not.
     std::vector<std::vector<int>> best;
     std::vector<int> all(nv);
@@ -121,7 +136,7 @@ bool planTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos,
     for (int k = std::max(1, (nv + vmax - 1) / vmax); k <= maxTiles;) {
         if (attempt(k, true)) {
             best = p.parts;
-            for (int j = k - 1; j > failedK && attempt(j, true); j--) best = p.parts;
+            for (int j = k - 1; fewest && j > failedK && attempt(j, true); j--) best = p.parts;
             break;
         }
         failedK = k;

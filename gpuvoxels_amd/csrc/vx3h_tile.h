@@ -27,10 +27,11 @@ struct TilePlan {
 // Cuts the voxels [0, nv) (lattice indices ijk, 3 per voxel) joined by links
 // (lneg, lpos, laxis per link) into compact blocks by recursive coordinate bisection,
 // each holding at most vmax owned + halo voxels and at most lax links per axis.
-// Tries a few target block sizes and keeps the plan with the fewest tiles.  False when
+// Tries a few target block sizes and keeps the plan with the fewest tiles, or without `fewest`
+// the first that fits, which has a few more at half the time.  False when
 // no plan has at most maxTiles tiles.
 bool planTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos, const int* laxis, int vmax, int lax,
-               int maxTiles, TilePlan* out);
+               int maxTiles, TilePlan* out, bool fewest = true);
 
 }  // namespace vx3
 #endif

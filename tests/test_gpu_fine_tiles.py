@@ -1,0 +1,81 @@
+"""Tiled simulations on the kernel with the links of all axes at once (taken when one launch
+holds their finer tiles and nothing else shares the chip) against the per-step kernels: the
+same bits, sampling steps and short launches included; and the way there and back as other
+simulations join and leave between calls."""
+import numpy as np
+import pytest
+
+from gpuvoxels_amd import _abi, engine, workloads
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac", "strain", "max_strain", "small_angle")
+
+
+def robot(seed, grid):
+    m = workloads.robot(np.random.default_rng(seed), grid=grid, steps=0)
+    m.materials[1].fixed = seed % 2
+    m.materials[2].mat_model, m.materials[2].fail_stress = _abi.MDL_LINEAR_FAIL, 800.0
+    return m
+
+
+def state(b, slots, models):
+    st = b.poll()
+    return [(b.read_state(s, nl=len(engine.topology(m)[0])), st[s]) for s, m in zip(slots, models)]
+
+
+def same(a, c):
+    for (x, sx), (y, sy) in zip(a, c):
+        assert sx.steps == sy.steps and sx.state == sy.state and sx.current_time == sy.current_time
+        for k in KEYS:
+            assert np.array_equal(x[k], y[k], equal_nan=True), k
+
+
+# two tiles; plans of 448 slots; as large as the shape takes; too many for one launch
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+@pytest.mark.parametrize("grids", [[14], [15, 27], [44, 44], [40, 40, 41, 42]])
+def test_equals_step_kernels(precision, grids):
+    models = [robot(i, g) for i, g in enumerate(grids)]
+    got = []
+    for noalloc in (False, True):
+        b = engine.Batch(precision=precision, path=_abi.PATH_AUTO, steps_per_launch=70)
+        slots = [b.admit(m) for m in models]
+        for n in (1, 2, 150):
+            (b.step_noalloc if noalloc else b.step)(n)
+        got.append(state(b, slots, models))
+        b.close()
+    same(*got)
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+def test_others_join_and_leave(precision):
+    big, small, plate = robot(3, 20), robot(4, 8), workloads.slab(20, 20, 2, steps=0)
+    more = [robot(5 + i, 43) for i in range(3)]
+    b = engine.Batch(precision=precision, path=_abi.PATH_AUTO)
+    s = b.admit(big)
+    b.step(20)                                  # finer tiles
+    fine = b.workgroups(s)
+    t = b.admit(small)
+    b.step(20)                                  # beside a one-workgroup simulation
+    coarse = b.workgroups(s)
+    assert 1 < coarse < fine
+    b.retire(t)
+    u = b.admit(plate)
+    b.step(20)                                  # beside the per-step kernels
+    assert b.workgroups(s) == coarse
+    b.retire(u)
+    b.step(20)
+    assert b.workgroups(s) == fine
+    v = [b.admit(m) for m in more]
+    b.step(20)                                  # larger tiles again, of either kernel
+    assert b.workgroups(s) < fine
+    for x in v:
+        b.retire(x)
+    b.step(20)
+    assert b.workgroups(s) == fine
+    c = engine.Batch(precision=precision, path=_abi.PATH_AUTO)
+    r = c.admit(big)
+    c.step_noalloc(120)
+    same(state(b, [s], [big]), state(c, [r], [big]))
+    b.close()
+    c.close()

@@ -48,8 +48,9 @@ def robots(n, grid):
 def check(models, precision, chunks):
     got = []
     for noalloc in (False, True):
-        b = engine.Batch(precision=precision)
+        b = engine.Batch(precision=precision, path=_abi.PATH_AUTO)
         slots = [b.admit(m) for m in models]
+        assert all(b.workgroups(s) == 1 for s in slots) or len(models) == 1   # (an edge's far side may be tiled)
         for n in chunks:
             (b.step_noalloc if noalloc else b.step)(n)
         st = b.poll()
