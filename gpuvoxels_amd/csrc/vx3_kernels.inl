@@ -679,6 +679,16 @@ __global__ void __launch_bounds__(256) k_col_list(DevBatch<real> b) {
 }
 
 
+// True only for pairs whose contact force is zero (pairContact's rel <= 0), without its square
+// root and divisions: most watched pairs most of the time.  The margin covers the rounding of
+// the contact distance and of the length (a few parts in 2^24); a distance whose square may have
+// lost bits to underflow decides nothing, nor does a NaN.
+__device__ __forceinline__ bool pairApart(real xi, real yi, real zi, real xj, real yj, real zj, float tfi, float tfj, real nom) {
+    const float ox = (float)(xj - xi), oy = (float)(yj - yi), oz = (float)(zj - zi);
+    const float reach = (float)nom * (tfi + tfj) * 0.625f, r2 = reach * reach;
+    return ox * ox + oy * oy + oz * oz > r2 * (1.0f + 0x1p-18f) && r2 > 1e-30f;
+}
+
 // Contact force of the pair (i, j), i the lower index, on voxel i: CVX_Collision::
 // updateContactForce (VX_Collision.cpp:41-56) from both voxels' pre-step position,
 // momentum and thermal factor.  Shared by the per-step and resident kernels.
@@ -718,6 +728,7 @@ struct Contacts {
             const int i = v < u ? v : u, j = v < u ? u : v;
             float fx, fy, fz;
             // both voxels' state from the contact snapshot (pre-step values)
+            if (pairApart(b->cpx[i], b->cpy[i], b->cpz[i], b->cpx[j], b->cpy[j], b->cpz[j], b->ctf[i], b->ctf[j], nom)) continue;
             pairContact(b->vmatTab[b->vmat[i]], b->vmatTab[b->vmat[j]], b->cpx[i], b->cpy[i], b->cpz[i], b->cpx[j], b->cpy[j],
                         b->cpz[j], b->cmx[i], b->cmy[i], b->cmz[i], b->cmx[j], b->cmy[j], b->cmz[j], b->ctf[i], b->ctf[j], nom,
                         fx, fy, fz);

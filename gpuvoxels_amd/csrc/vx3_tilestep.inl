@@ -319,27 +319,47 @@ struct TsContacts {
     int v, v0, start, count, mat;
     real x, y, z, mx, my, mz, nom;
     float tf;
+    // Partners whose loads are in flight together, those apart left after their distance.  FP32,
+    // 300 balls with 17,800 pairs: 33 us a step, 45 one at a time and every pair computed.  FP64:
+    // either takes registers that spill outside this loop too (2,048 balls 147 us, 141 without).
+    static constexpr int AT_ONCE = sizeof(real) == 8 ? 1 : 4;
     template <typename T> __device__ __forceinline__ void subtract(V3<T>& force) const {
 #pragma unroll 1
-        for (int k = 0; k < count; k++) {
-            const int u = b->nbList[start + k];
-            const int q = o2p[u - v0];
-            const int rec = q >> VX3_TS_SLOT_BITS, s = q & ((1 << VX3_TS_SLOT_BITS) - 1);
-            char* C = tsState(*ts, rec, ts->par);
-            const real ux = row<real>(C, TsS::VR, s), uy = row<real>(C, TsS::VR + TsS::RR, s), uz = row<real>(C, TsS::VR + 2 * TsS::RR, s);
-            const real nx = row<real>(C, TsS::VR + 7 * TsS::RR, s), ny = row<real>(C, TsS::VR + 8 * TsS::RR, s),
-                       nz = row<real>(C, TsS::VR + 9 * TsS::RR, s);
-            const float tu = row<float>(C, TsS::VF, s);
-            const VoxMatDev& mu = vm[row<unsigned>(tsStat(*ts, rec), TsA::ST, s) & 15];
-            const VoxMatDev& mv = vm[mat];
-            float fx, fy, fz;
-            if (v < u)
-                pairContact(mv, mu, x, y, z, ux, uy, uz, mx, my, mz, nx, ny, nz, tf, tu, nom, fx, fy, fz);
-            else {
-                pairContact(mu, mv, ux, uy, uz, x, y, z, nx, ny, nz, mx, my, mz, tu, tf, nom, fx, fy, fz);
-                fx = -fx; fy = -fy; fz = -fz;
+        for (int k0 = 0; k0 < count; k0 += AT_ONCE) {   // (past the last: the last again, left out)
+            int us[AT_ONCE], qs[AT_ONCE];
+            real px[AT_ONCE], py[AT_ONCE], pz[AT_ONCE];
+            float tfs[AT_ONCE];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; i++) us[i] = b->nbList[start + (k0 + i < count ? k0 + i : count - 1)];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; i++) qs[i] = o2p[us[i] - v0];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; i++) {
+                char* C = tsState(*ts, qs[i] >> VX3_TS_SLOT_BITS, ts->par);
+                const int s = qs[i] & ((1 << VX3_TS_SLOT_BITS) - 1);
+                px[i] = row<real>(C, TsS::VR, s); py[i] = row<real>(C, TsS::VR + TsS::RR, s); pz[i] = row<real>(C, TsS::VR + 2 * TsS::RR, s);
+                tfs[i] = row<float>(C, TsS::VF, s);
             }
-            force.x -= (T)fx; force.y -= (T)fy; force.z -= (T)fz;
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; i++) {
+                if (AT_ONCE > 1 && (k0 + i >= count || pairApart(x, y, z, px[i], py[i], pz[i], tf, tfs[i], nom))) continue;
+                const int u = us[i], rec = qs[i] >> VX3_TS_SLOT_BITS, s = qs[i] & ((1 << VX3_TS_SLOT_BITS) - 1);
+                char* C = tsState(*ts, rec, ts->par);
+                const real ux = px[i], uy = py[i], uz = pz[i];
+                const real nx = row<real>(C, TsS::VR + 7 * TsS::RR, s), ny = row<real>(C, TsS::VR + 8 * TsS::RR, s),
+                           nz = row<real>(C, TsS::VR + 9 * TsS::RR, s);
+                const float tu = tfs[i];
+                const VoxMatDev& mu = vm[row<unsigned>(tsStat(*ts, rec), TsA::ST, s) & 15];
+                const VoxMatDev& mv = vm[mat];
+                float fx, fy, fz;
+                if (v < u)
+                    pairContact(mv, mu, x, y, z, ux, uy, uz, mx, my, mz, nx, ny, nz, tf, tu, nom, fx, fy, fz);
+                else {
+                    pairContact(mu, mv, ux, uy, uz, x, y, z, nx, ny, nz, mx, my, mz, tu, tf, nom, fx, fy, fz);
+                    fx = -fx; fy = -fy; fz = -fz;
+                }
+                force.x -= (T)fx; force.y -= (T)fy; force.z -= (T)fz;
+            }
         }
     }
 };
