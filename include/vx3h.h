@@ -399,7 +399,8 @@ vx3h_status vx3h_batch_kernel_times(vx3h_batch* b, int n_steps, double* avg_ms);
 
 /* Which kernels step a simulation (no counterpart in the reference, which has one
  * path): *workgroups = 0 for the per-step kernels, 1 for one workgroup of the resident
- * kernel, n > 1 for n tiles of the tiled resident kernel. */
+ * kernel, n > 1 for n tiles of the tiled resident kernel (as of the last stepping call: a
+ * simulation that has the device to itself runs as more, smaller tiles). */
 vx3h_status vx3h_sim_workgroups(vx3h_batch* b, int slot, int* workgroups);
 
 /* Launch timing of ordinary stepping (no counterpart in the reference): while
