@@ -84,7 +84,7 @@ hipError_t launchTileStep(const DevBatch<VX_REAL>& b, const TsArgs& ts, hipStrea
 }
 
 void launchDt(const DevBatch<VX_REAL>& b, hipStream_t s, int s0, int s1) {
-    if (s1 > s0) hipLaunchKernelGGL(VX_NS::k_dt, dim3(s1 - s0), dim3(256), 0, s, b, s0, s1);
+    if (s1 > s0) hipLaunchKernelGGL(VX_NS::k_dt, dim3(s1 - s0), dim3(VX3_DT_BLOCK), 0, s, b, s0, s1);
 }
 
 }  // namespace vx3
