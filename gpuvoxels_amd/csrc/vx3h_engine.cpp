@@ -24,6 +24,7 @@
 #include "vx3_launch.h"
 #include "vx3h_build.h"
 #include "vx3h_internal.h"
+#include "vx3h_pool.h"
 #include "vx3h_steptile.h"
 #include "vx3h_tile.h"
 
@@ -70,39 +71,9 @@ struct ArrSpec {
     bool strided;
 };
 
-struct Range { int start, len; };
-
-struct RangeAlloc {
-    std::map<int, int> freeRanges;   // start -> length
-    int hi = 0;
-    int alloc(int n, int cap, bool& grow) {
-        grow = false;
-        for (auto it = freeRanges.begin(); it != freeRanges.end(); ++it) {
-            if (it->second >= n) {
-                int s = it->first, len = it->second;
-                freeRanges.erase(it);
-                if (len > n) freeRanges[s + n] = len - n;
-                return s;
-            }
-        }
-        int s = hi;
-        hi += n;
-        if (hi > cap) grow = true;
-        return s;
-    }
-    void release(int s, int n) {
-        if (n <= 0) return;
-        freeRanges[s] = n;
-        auto it = freeRanges.find(s);
-        auto nx = std::next(it);
-        if (nx != freeRanges.end() && it->first + it->second == nx->first) { it->second += nx->second; freeRanges.erase(nx); }
-        if (it != freeRanges.begin()) {
-            auto pv = std::prev(it);
-            if (pv->first + pv->second == it->first) { pv->second += it->second; freeRanges.erase(it); it = pv; }
-        }
-        if (it->first + it->second == hi) { hi = it->first; freeRanges.erase(it); }
-    }
-};
+// Tile tables' ranges in the tile pools: tile slots, tile links, exchange records, tiles
+// (tiles 0: not placed).
+struct TilePlace { int v0 = 0, vN = 0, l0 = 0, lN = 0, x0 = 0, xN = 0, p0 = 0, tiles = 0; };
 
 struct SlotHost {
     bool used = false;
@@ -113,9 +84,8 @@ struct SlotHost {
     int tiles = 0;               // > 0: runs on the tiled resident kernel as this many workgroups
     TilePlan tplan, fplan;       // its tiles (sim-local): for the axis-by-axis kernel, and finer ones (planned when first
                                  // used) for the kernel with the links of all axes at once
-    bool fine = false;           // the device tables are the finer ones'
     int fineSlots = 0;           // owned and halo voxels of a tile that fplan was planned for (0: not yet)
-    int tv0 = 0, tvN = 0, tl0 = 0, tlN = 0, tx0 = 0, txN = 0, tp0 = 0;   // its ranges in the tile pools
+    TilePlace tplace, fplace;    // their tables: the first from admission on, the finer ones beside them once used
     bool oneTile = false;        // a one-workgroup simulation with one-tile tables in the pools
     int axisLinks = 0;           // links on its busiest axis
     std::vector<TsTile> stepTiles;   // steps on the fused per-step kernel as these tiles
@@ -419,12 +389,12 @@ vx3h_status growArrays(vx3h_batch* b, std::vector<ArrSpec>& arrs, int& cap, int 
     return VX3H_OK;
 }
 
-vx3h_status poolAlloc(vx3h_batch* b, DevPool& p, int n, int& start) {
-    bool grow = false;
-    start = p.ra.alloc(n, p.cap, grow);
-    if (!grow) return VX3H_OK;
+// Enlarges a pool's arrays to hold its ranges.  An array that cannot be allocated leaves those
+// before it enlarged, which the capacity does not count yet.
+vx3h_status poolGrow(vx3h_batch* b, DevPool& p) {
     const int ncap = std::max(p.ra.hi, std::max(2 * p.cap, p.minCap));
     HIPCHK(hipStreamSynchronize(b->stream));
+    b->layout++;
     for (auto& a : p.arrs) {
         void* np = nullptr;
         HIPCHK(hipMalloc(&np, (size_t)ncap * a.second));
@@ -436,8 +406,11 @@ vx3h_status poolAlloc(vx3h_batch* b, DevPool& p, int n, int& start) {
         *a.first = np;
     }
     p.cap = ncap;
-    b->layout++;
     return VX3H_OK;
+}
+
+vx3h_status poolAlloc(vx3h_batch* b, DevPool& p, int n, int& start) {
+    return takeRange(p, n, start, [&](DevPool& q) { return poolGrow(b, q); });
 }
 
 template <typename E> vx3h_status uploadTable(vx3h_batch* b, void*& dptr, size_t& cap, const std::vector<E>& v) {
@@ -643,11 +616,45 @@ bool absorbable(const vx3h_batch* b, size_t i) { return i < b->shapes.size() || 
 // grows a device array to at least n elements (contents not kept)
 template <typename T> vx3h_status growDev(T** p, size_t* cap, size_t n) {
     if (n <= *cap) return VX3H_OK;
+    const size_t c = std::max(n, *cap + *cap / 2);
     if (*p) HIPCHK(hipFree(*p));
     *p = nullptr;
-    const size_t c = std::max(n, *cap + *cap / 2);
+    *cap = 0;
     HIPCHK(hipMalloc((void**)p, c * sizeof(T)));
     *cap = c;
+    return VX3H_OK;
+}
+
+void releaseTiles(vx3h_batch* b, TilePlace& t) {
+    if (t.tiles) {
+        b->tileSlotPool.ra.release(t.v0, t.vN);
+        b->tileLinkPool.ra.release(t.l0, t.lN);
+        b->tileXchPool.ra.release(t.x0, t.xN);
+        b->tilePartPool.ra.release(t.p0, t.tiles);
+    }
+    t = TilePlace();
+}
+
+// Puts a plan's tile tables into the pools; after an error they are not placed.
+vx3h_status placeTiles(vx3h_batch* b, const TilePlan& p, TilePlace* out) {
+    TilePlace t;
+    t.vN = std::max(1, (int)p.vox.size());
+    t.lN = std::max(1, (int)p.link.size());
+    t.xN = std::max(1, p.nPub);
+    t.tiles = (int)p.tiles.size();
+    DevPool* const pools[4] = {&b->tileSlotPool, &b->tileLinkPool, &b->tileXchPool, &b->tilePartPool};
+    const int n[4] = {t.vN, t.lN, t.xN, t.tiles};
+    int* const start[4] = {&t.v0, &t.l0, &t.x0, &t.p0};
+    vx3h_status st = takeRanges(pools, n, start, [&](DevPool& q) { return poolGrow(b, q); });
+    if (st) return st;
+    if ((st = upload(b, b->dTileVox + t.v0, p.vox.data(), p.vox.size() * 4)) ||
+        (st = upload(b, b->dTileXidx + t.v0, p.xidx.data(), p.xidx.size() * 4)) ||
+        (st = upload(b, b->dTileLink + t.l0, p.link.data(), p.link.size() * 4)) ||
+        (st = upload(b, b->dTileEnds + t.l0, p.ends.data(), p.ends.size() * 4))) {
+        releaseTiles(b, t);
+        return st;
+    }
+    *out = t;
     return VX3H_OK;
 }
 
@@ -658,53 +665,20 @@ vx3h_status ensureOneTile(vx3h_batch* b, int s) {
     if (sh.oneTile) return VX3H_OK;
     TileDesc d{};
     d.tile = 0; d.nTiles = 1; d.vOff = 0; d.nOwn = sh.nv; d.nHalo = 0; d.lOff = 0; d.nLinks = sh.nl;
-    std::vector<int> vox(sh.nv), xidx(sh.nv, -1), link(sh.nl), ends(sh.nl);
-    for (int i = 0; i < sh.nv; i++) vox[i] = i;
+    TilePlan p;
+    p.vox.resize(sh.nv); p.xidx.assign(sh.nv, -1); p.link.resize(sh.nl); p.ends.resize(sh.nl);
+    for (int i = 0; i < sh.nv; i++) p.vox[i] = i;
     for (int l = 0; l < sh.nl; l++) {
-        link[l] = l | (int)0x80000000u;
-        ends[l] = sh.lneg[l] | (sh.lpos[l] << 16);
+        p.link[l] = l | (int)0x80000000u;
+        p.ends[l] = sh.lneg[l] | (sh.lpos[l] << 16);
     }
-    sh.tvN = std::max(1, sh.nv);
-    sh.tlN = std::max(1, sh.nl);
-    sh.txN = 1;
-    vx3h_status st;
-    if ((st = poolAlloc(b, b->tileSlotPool, sh.tvN, sh.tv0)) || (st = poolAlloc(b, b->tileLinkPool, sh.tlN, sh.tl0)) ||
-        (st = poolAlloc(b, b->tileXchPool, sh.txN, sh.tx0)) || (st = poolAlloc(b, b->tilePartPool, 1, sh.tp0)))
-        return st;
-    if ((st = upload(b, b->dTileVox + sh.tv0, vox.data(), vox.size() * 4)) ||
-        (st = upload(b, b->dTileXidx + sh.tv0, xidx.data(), xidx.size() * 4)) ||
-        (st = upload(b, b->dTileLink + sh.tl0, link.data(), link.size() * 4)) ||
-        (st = upload(b, b->dTileEnds + sh.tl0, ends.data(), ends.size() * 4)))
-        return st;
-    sh.tplan.tiles.assign(1, d);
+    p.tiles.assign(1, d);
+    p.nPub = 0;
+    if (vx3h_status st = placeTiles(b, p, &sh.tplace)) return st;
+    sh.tplan.tiles = std::move(p.tiles);
     sh.tplan.nPub = 0;
     sh.oneTile = true;
     return VX3H_OK;
-}
-
-// Puts a simulation's tile tables into the pools.
-vx3h_status placeTiles(vx3h_batch* b, SlotHost& sh, const TilePlan& p) {
-    vx3h_status st;
-    sh.tvN = (int)p.vox.size();
-    sh.tlN = std::max(1, (int)p.link.size());
-    sh.txN = std::max(1, p.nPub);
-    sh.tiles = (int)p.tiles.size();
-    if ((st = poolAlloc(b, b->tileSlotPool, sh.tvN, sh.tv0)) || (st = poolAlloc(b, b->tileLinkPool, sh.tlN, sh.tl0)) ||
-        (st = poolAlloc(b, b->tileXchPool, sh.txN, sh.tx0)) || (st = poolAlloc(b, b->tilePartPool, sh.tiles, sh.tp0)))
-        return st;
-    if ((st = upload(b, b->dTileVox + sh.tv0, p.vox.data(), p.vox.size() * 4)) ||
-        (st = upload(b, b->dTileXidx + sh.tv0, p.xidx.data(), p.xidx.size() * 4)) ||
-        (st = upload(b, b->dTileLink + sh.tl0, p.link.data(), p.link.size() * 4)) ||
-        (st = upload(b, b->dTileEnds + sh.tl0, p.ends.data(), p.ends.size() * 4)))
-        return st;
-    return VX3H_OK;
-}
-
-void releaseTiles(vx3h_batch* b, SlotHost& sh) {
-    b->tileSlotPool.ra.release(sh.tv0, sh.tvN);
-    b->tileLinkPool.ra.release(sh.tl0, sh.tlN);
-    b->tileXchPool.ra.release(sh.tx0, sh.txN);
-    b->tilePartPool.ra.release(sh.tp0, sh.tiles);
 }
 
 // Whether the tiled simulations step as finer tiles on the kernel with the links of all axes at
@@ -740,29 +714,22 @@ vx3h_status chooseTiles(vx3h_batch* b) {
             if (!planTiles(sh.nv, sh.ijk.data(), sh.nl, sh.lneg.data(), sh.lpos.data(), axis.data(), slots, b->fineShape.links / 3,
                            b->fineCap, &p, false))
                 p = TilePlan();
-            if (sh.fine) {   // its tables are the old plan's
-                HIPCHK(hipStreamSynchronize(b->stream));
-                releaseTiles(b, sh);
-                sh.fine = false;
-                if (vx3h_status st = placeTiles(b, sh, sh.tplan)) return st;
-            }
+            HIPCHK(hipStreamSynchronize(b->stream));   // launches that read the old plan's tables
+            releaseTiles(b, sh.fplace);
             sh.fplan = std::move(p);
             sh.fineSlots = slots;
         }
         tiles += sh.fplan.tiles.size();
         fine = sh.fplan.tiles.size() > 1 && tiles <= cap;
     }
-    b->fine = fine;
-    bool synced = false;
-    for (int s : b->tiledSims) {
-        SlotHost& sh = b->slots[s];
-        if (sh.fine == fine) continue;
-        if (!synced) HIPCHK(hipStreamSynchronize(b->stream));   // launches that read the tables
-        synced = true;
-        releaseTiles(b, sh);
-        sh.fine = fine;
-        if (vx3h_status st = placeTiles(b, sh, fine ? sh.fplan : sh.tplan)) return st;
+    for (size_t i = 0; fine && i < b->tiledSims.size(); i++) {
+        SlotHost& sh = b->slots[b->tiledSims[i]];
+        if (sh.fplace.tiles || placeTiles(b, sh.fplan, &sh.fplace) == VX3H_OK) continue;
+        fine = false;   // no device memory for them: the larger tiles stay
+        (void)hipGetLastError();
     }
+    b->fine = fine;
+    for (int s : b->tiledSims) b->slots[s].tiles = (int)(fine ? b->slots[s].fplan : b->slots[s].tplan).tiles.size();
     return VX3H_OK;
 }
 
@@ -809,15 +776,17 @@ vx3h_status syncTiles(vx3h_batch* b) {
         vx3h_batch::TileGroup g{(int)T.size(), 0, syncTot, 0};
         for (int s : bin) {
             const SlotHost& sh = b->slots[s];
-            const TilePlan& plan = sh.fine ? sh.fplan : sh.tplan;
+            const bool fine = b->fine && sh.tiles;
+            const TilePlan& plan = fine ? sh.fplan : sh.tplan;
+            const TilePlace& at = fine ? sh.fplace : sh.tplace;
             for (TileDesc d : plan.tiles) {
                 d.sim = s;
-                d.vOff += sh.tv0;
-                d.lOff += sh.tl0;
-                d.xOff = sh.tx0 * 2 * VX3_XCH_STRIDE;
+                d.vOff += at.v0;
+                d.lOff += at.l0;
+                d.xOff = at.x0 * 2 * VX3_XCH_STRIDE;
                 d.xPar = VX3_XCH_STRIDE * plan.nPub;
                 d.cOff = g.nSync;
-                d.pOff = sh.tp0 * 8;
+                d.pOff = at.p0 * 8;
                 T.push_back(d);
             }
             g.count += tilesOf(s);
@@ -842,12 +811,18 @@ vx3h_status stepCtl(vx3h_batch* b) {
     TsArgs& t = b->ts;
     if (b->stepCtlCap == b->stepCtlPool.cap) return VX3H_OK;
     const size_t c = b->stepCtlPool.cap;
+    TsCtl* ctl = nullptr;   // both before either is replaced: simulations that have theirs go on after an error
+    TsReport* report = nullptr;
+    HIPCHK(hipMalloc((void**)&ctl, c * 2 * sizeof(TsCtl)));
+    if (hipMalloc((void**)&report, c * 2 * sizeof(TsReport)) != hipSuccess) {
+        hipFree(ctl);
+        FAILV(VX3H_ENOMEM, "device memory too small for the step tiles' control states");
+    }
     HIPCHK(hipStreamSynchronize(b->stream));
-    b->stepCtlCap = 0;
-    if (t.ctl) { HIPCHK(hipFree(t.ctl)); t.ctl = nullptr; }
-    if (t.report) { HIPCHK(hipFree(t.report)); t.report = nullptr; }
-    HIPCHK(hipMalloc((void**)&t.ctl, c * 2 * sizeof(TsCtl)));
-    HIPCHK(hipMalloc((void**)&t.report, c * 2 * sizeof(TsReport)));
+    if (t.ctl) HIPCHK(hipFree(t.ctl));
+    if (t.report) HIPCHK(hipFree(t.report));
+    t.ctl = ctl;
+    t.report = report;
     HIPCHK(hipMemsetAsync(t.report, 0, c * 2 * sizeof(TsReport), b->stream));   // report numbers start at 1
     b->stepCtlCap = t.ctlCap = (int)c;
     b->layout++;
@@ -1789,8 +1764,10 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     sh.tg0 = tg0; sh.nTg = nTg;
     sh.at0 = at0; sh.ap0 = ap0; sh.apN = apN;
     if (tiles) {
-        sh.tplan = std::move(tplan);
-        if (vx3h_status st = placeTiles(b, sh, sh.tplan)) return st;
+        if (vx3h_status st = placeTiles(b, tplan, &sh.tplace)) return st;
+        sh.tiles = tiles;
+        sh.tplan.tiles = std::move(tplan.tiles);   // the descriptors stay on the host
+        sh.tplan.nPub = tplan.nPub;
         b->tiledSims.push_back(s);
         b->tileDirty = true;
     } else if (shape >= 0) {   // the kernel variant with contacts for a simulation with collisions
@@ -2296,6 +2273,7 @@ namespace {
 // A fresh range of `need` entries for one simulation in a pool (the old range is released).
 vx3h_status regrow(vx3h_batch* b, DevPool& p, int& start, int& len, int need) {
     p.ra.release(start, len);
+    len = 0;   // (after an error it has none)
     vx3h_status st = poolAlloc(b, p, need, start);
     if (st) return st;
     len = need;
@@ -2480,7 +2458,7 @@ extern "C" vx3h_status vx3h_sim_retire(vx3h_batch* b, int slot) {
     }
     if (sh.tiles) {
         b->tiledSims.erase(std::remove(b->tiledSims.begin(), b->tiledSims.end(), slot), b->tiledSims.end());
-        releaseTiles(b, sh);
+        releaseTiles(b, sh.fplace);
         b->tileDirty = true;
     } else if (sh.shape >= 0) {
         auto& L = b->resLists[sh.shape];
@@ -2492,12 +2470,7 @@ extern "C" vx3h_status vx3h_sim_retire(vx3h_batch* b, int slot) {
         releaseStep(b, sh);
         b->stepDirty = b->tileDirty = true;
     } else { b->nStreamSims--; b->tileDirty = true; }
-    if (sh.oneTile) {
-        b->tileSlotPool.ra.release(sh.tv0, sh.tvN);
-        b->tileLinkPool.ra.release(sh.tl0, sh.tlN);
-        b->tileXchPool.ra.release(sh.tx0, sh.txN);
-        b->tilePartPool.ra.release(sh.tp0, 1);
-    }
+    releaseTiles(b, sh.tplace);   // (a one-workgroup simulation's one tile too)
     b->bytesUsed -= sh.bytes;
     sh = SlotHost();
     b->db.vHi = b->va.hi;
