@@ -212,7 +212,7 @@ struct vx3h_batch {
     DevPool stepTilePool, stepPhasePool, stepO2pPool, stepCtlPool;
     int stepCtlCap = 0;                          // control states allocated
     int stepPar = 0;                             // parity of the next step of the call
-    unsigned stepSeq = 1;                        // report numbers used so far
+    TsNumbers stepNumbers;
     hipGraphExec_t stepGraphExec = nullptr;
     hipGraph_t stepGraph = nullptr;
     int stepGraphSteps = 0;
@@ -947,13 +947,16 @@ vx3h_status syncStep(vx3h_batch* b) {
     return VX3H_OK;
 }
 
-// n launches of the fused kernel (what: TS_LOAD and TS_STORE once, around a call's steps)
+// n launches of the fused kernel (what: TS_LOAD and TS_STORE once, around a call's steps; the
+// load's n: the steps of the call)
 vx3h_status launchStepTiles(vx3h_batch* b, int what, int n) {
     TsArgs a = b->ts;
     if (what == TS_LOAD) {
         b->stepPar = 0;
-        a.seq0 = b->stepSeq;
-        b->stepSeq++;
+        bool restart;
+        a.seq0 = b->stepNumbers.take(1u + (unsigned)n, &restart);
+        if (restart) HIPCHK(hipMemsetAsync(a.report, 0, (size_t)b->stepCtlCap * 2 * sizeof(TsReport), b->stream));
+        n = 1;
     }
     for (int i = 0; i < n; i++) {
         a.par = b->stepPar;
@@ -968,7 +971,6 @@ vx3h_status launchStepTiles(vx3h_batch* b, int what, int n) {
 
 // n steps of the fused kernel, in graphs of up to 32 (an even number, from parity 0)
 vx3h_status runStepTiles(vx3h_batch* b, int n) {
-    b->stepSeq += (unsigned)n;
     if (!b->cfg.use_graph) return launchStepTiles(b, TS_STEP, n);
     vx3h_status st;
     if (n > 0 && b->stepPar) {
@@ -1865,7 +1867,7 @@ extern "C" vx3h_status vx3h_batch_step(vx3h_batch* b, int n_steps) {
         }
         if (!st && fused && !plain) {
             if (!loaded) {
-                st = launchStepTiles(b, TS_LOAD, 1);
+                st = launchStepTiles(b, TS_LOAD, n_steps - done);
                 loaded = true;
             }
             if (!st) st = runStepTiles(b, c);
@@ -2109,9 +2111,8 @@ extern "C" vx3h_status vx3h_batch_kernel_times(vx3h_batch* b, int n_steps, doubl
         hipEvent_t e0, e1;
         HIPCHK(hipEventCreate(&e0));
         HIPCHK(hipEventCreate(&e1));
-        if ((st = launchStepTiles(b, TS_LOAD, 1))) return st;
+        if ((st = launchStepTiles(b, TS_LOAD, n_steps))) return st;
         HIPCHK(hipEventRecord(e0, b->stream));
-        b->stepSeq += (unsigned)n_steps;
         st = launchStepTiles(b, TS_STEP, n_steps);
         HIPCHK(hipEventRecord(e1, b->stream));
         const vx3h_status ls = launchStepTiles(b, TS_STORE, 1);

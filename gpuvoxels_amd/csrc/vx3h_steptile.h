@@ -2,6 +2,7 @@
 #ifndef VX3H_STEPTILE_H
 #define VX3H_STEPTILE_H
 #include <cstddef>
+#include <cstdint>
 #include <vector>
 #include "vx3_types.h"
 
@@ -26,6 +27,21 @@ struct StepTilePlan {
 // for an empty simulation or a lattice of more than 2^16 along an axis.
 bool planStepTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos, const int* vlinks,
                    const char* interior, StepTilePlan* out);
+
+// The numbers under which the fused kernel's steps report (TsReport).  Report words are matched
+// by number and never cleared one by one, so a number is used once: when a call's would pass the
+// largest, all words have to be cleared and the numbers start over.
+struct TsNumbers {
+    unsigned next = 1;   // (0: a cleared word's)
+    // the first of n numbers (1 <= n <= 2^31), one after another; *restart: clear the words first
+    unsigned take(unsigned n, bool* restart) {
+        *restart = next == 0 || n - 1 > UINT32_MAX - next;
+        if (*restart) next = 1;
+        const unsigned first = next;
+        next += n;
+        return first;
+    }
+};
 
 }  // namespace vx3
 #endif
