@@ -21,7 +21,7 @@
 // A step that cannot be taken (a collision table too small: TsReport::grow) or not as a whole
 // (a diverged link: its voxels do not move) is only known once every tile has run: the
 // control step then leaves the old copy current (SC_TSPARV, SC_TSPARL), so nothing has
-// happened, or only the link pass has.  A running simulation's current copies are always
+// happened but for the partner lists, or only the link pass has.  A running simulation's current copies are always
 // those of the launch's parity, so a tile reads its state without waiting for the control
 // words.
 //
@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) k_ts_load(DevBatch<real> b, TsAr
             row<float>(C, TsS::LF + 2 * a * TsS::R4, i) = b.maxStrain[g];
             row<float>(C, TsS::LF + (2 * a + 1) * TsS::R4, i) = b.strainOffset[g];
             row<unsigned char>(C, TsS::LB + a * VX3_TS_OWN, i) = (unsigned char)b.lflags[g];
-            row<float>(A, TsA::LS + a * TsA::R4, i) = b.strain[g];
+            row<float>(C, TsS::LS + a * TsS::R4, i) = b.strain[g];
         }
     }
     if (col) {
@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) k_ts_store(DevBatch<real> b, TsA
             b.maxStrain[g] = row<float>(L, TsS::LF + 2 * a * TsS::R4, i);
             if (!b.lmatTab[b.lmeta[g] >> 2].linear) b.strainOffset[g] = row<float>(L, TsS::LF + (2 * a + 1) * TsS::R4, i);
             b.lflags[g] = lb;
-            b.strain[g] = row<float>(A, TsA::LS + a * TsA::R4, i);
+            b.strain[g] = row<float>(L, TsS::LS + a * TsS::R4, i);
         }
     }
     if (td.tile == 0 && tid == 0) {   // the other tiles read no field that changes here
@@ -969,7 +969,7 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) __attribute__((amdgpu_waves_per_
             V3<real> fn, mn_;
             float en = 0;
             if (mn.fixed && mp.fixed) {   // not computed: its loads are never read, its strain stays zero
-                if (mine) ls.strain = row<float>(A + a * TsA::R4, TsA::LS, j);
+                if (mine) ls.strain = row<float>(C + a * TsS::R4, TsS::LS, j);
                 if (vp < td.nOwn) sEnd[vp] = 0;
             } else {
                 const real restLength = (real)0.5 * (nom * (real)sF[vn] + nom * (real)sF[vp]);
@@ -1036,7 +1036,7 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) __attribute__((amdgpu_waves_per_
                 row<float>(F, TsS::LF, j) = ls.maxStrain;
                 if (!mat.linear) row<float>(F, TsS::LF + TsS::R4, j) = ls.strainOffset;
                 row<unsigned char>(D + a * VX3_TS_OWN, TsS::LB, j) = (unsigned char)ls.flags;
-                row<float>(A + a * TsA::R4, TsA::LS, j) = ls.strain;
+                row<float>(D + a * TsS::R4, TsS::LS, j) = ls.strain;
             }
         }
         if (a == 2) break;

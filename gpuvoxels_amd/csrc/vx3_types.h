@@ -214,7 +214,9 @@ struct TsTile {
 #define VX3_TS_SLOT_BITS 9
 
 // A tile record: rows of VX3_TS_OWN elements, one per owned slot.  TsStat (byte offsets) is
-// written at admission up to ST_END; the rest and TsState belong to a call.
+// written at admission up to ST_END; the rest and TsState belong to a call.  What a step that is
+// not taken (TsReport::grow) may have overwritten in TsStat, the lists and what goes with them,
+// is rebuilt by the step that is taken in its place.
 struct TsStat {
     static constexpr int R4 = 4 * VX3_TS_OWN;
     static constexpr int ST = 0;               // voxel material | phase << 4 | external << 10 | link material of axis a << (12 + 4a)
@@ -226,8 +228,7 @@ struct TsStat {
     static constexpr int IJK = LINK + 3 * R4;  // row of pairs of words: lattice index from the simulation's lowest, x | y << 16
                                                // and z | (121 x + 11 y + z) << 16 (modulo 2^16; see NearBitTable's index)
     static constexpr int ST_END = IJK + 2 * R4;
-    static constexpr int LS = ST_END;          // 3 rows: strain of the last step
-    static constexpr int LW = LS + 3 * R4;     // 3 rows: position at the last list rebuild
+    static constexpr int LW = ST_END;          // 3 rows: position at the last list rebuild
     static constexpr int NBC = LW + 3 * R4, NBS = NBC + R4;   // partner list: entries, start in nbList
     static constexpr int BYTES = (NBS + R4 + 255) / 256 * 256;
 };
@@ -237,7 +238,8 @@ template <int REAL> struct TsState {   // one of the two copies; REAL = bytes of
     static constexpr int LR = 13 * RR;         // per axis 9 rows: previous pos2, angle2v, angle1v (large-angle links only)
     static constexpr int VF = LR + 27 * RR;    // 4 rows: thermal factor, Poisson strain
     static constexpr int LF = VF + 4 * R4;     // per axis 2 rows: maxStrain, strainOffset (the latter: non-linear materials only)
-    static constexpr int VI = LF + 6 * R4;     // voxel flags
+    static constexpr int LS = LF + 6 * R4;     // per axis: strain of the last step
+    static constexpr int VI = LS + 3 * R4;     // voxel flags
     static constexpr int LB = VI + R4;         // 3 rows of bytes: LF_* bits
     static constexpr int BYTES = (LB + 3 * VX3_TS_OWN + 255) / 256 * 256;
 };

@@ -101,6 +101,7 @@ struct SlotHost {
     size_t bytes = 0;
     // collision pools: neighbour lists, hash buckets, nearby lists
     int nb0 = 0, nbN = 0, h0 = 0, hN = 0, near0 = 0, nearN = 0, c0 = 0;   // hN in buckets (whole blocks)
+    int listsLost = -1;          // >= 0: a rebuild that its table was too small for, after this many, broke the lists off
     int tg0 = 0, nTg = 0;        // close pairs: range of the sim's target voxels in tgtList
     int at0 = 0, ap0 = 0, apN = 0;   // attach scratch ranges (attCand: 2*nv; attPair: apN)
     // history records: topology and link constants of the sim, palette in order
@@ -2358,6 +2359,7 @@ vx3h_status growCollisionTables(vx3h_batch* b, std::vector<SimCtl>& ctl) {
             b->layout++;
         }
         if (c.nbNeed > c.nbCap) {
+            sh.listsLost = c.rebuilds;
             if ((st = regrow(b, b->nbPool, sh.nb0, sh.nbN, std::max(2 * sh.nbN, c.nbNeed + c.nbNeed / 2)))) return st;
             c.nb0 = sh.nb0;
             c.nbCap = sh.nbN;
@@ -2488,6 +2490,11 @@ extern "C" vx3h_status vx3h_sim_collision_pairs(vx3h_batch* b, int slot, int* pa
     const SlotHost& sh = b->slots[slot];
     *n = 0;
     if (!sh.nbN || !sh.nv) return VX3H_OK;
+    // a rebuild that ran out of table has overwritten some of the lists before it
+    SimCtl c;
+    HIPCHK(hipMemcpy(&c, b->db.sims + slot, sizeof(SimCtl), hipMemcpyDeviceToHost));
+    if (((c.flags & SC_COL_GROW) && c.nbNeed > c.nbCap) || c.rebuilds == sh.listsLost)
+        FAILV(VX3H_EDEVICE, "collision lists incomplete: their table was too small, the next step after vx3h_batch_poll rebuilds them");
     std::vector<int> st(sh.nv), cnt(sh.nv), fl(sh.nv);
     HIPCHK(hipMemcpy(st.data(), b->db.nbStart + sh.v0, sh.nv * 4, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(cnt.data(), b->db.nbCount + sh.v0, sh.nv * 4, hipMemcpyDeviceToHost));

@@ -419,7 +419,8 @@ vx3h_status vx3h_calib_copy(int device, size_t bytes, int reps, double* ms_per_c
 /* Collision pairs a simulation currently watches, as sim-local voxel index pairs
  * (i < j) in ascending order -- CVoxelyze's collision list after its last
  * regeneration (Voxelyze3/src/old/Voxelyze.cpp:726-751).  pairs holds 2*cap ints and
- * may be NULL to query *n. */
+ * may be NULL to query *n.  VX3H_EDEVICE from the time a regeneration stops for a larger
+ * table until the simulation's next step: there is no complete list then. */
 vx3h_status vx3h_sim_collision_pairs(vx3h_batch* b, int slot, int* pairs, int cap, int* n);
 
 /* ---------------------------------------------------------------- autotuner

@@ -146,3 +146,46 @@ def test_beside_resident_and_retired():
         for k in ("pos", "orient", "lin_mom", "ang_mom", "flags"):
             assert np.array_equal(got[k], ref[k]), k
     b.close()
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+def test_standing_still_for_a_table_changes_nothing(precision):
+    """A simulation that stops within a call because its lists outgrow their table, in some tiles
+    but not in others: until it goes on its state, link strains included, is that of its last
+    step, and there is no pair list."""
+    m = workloads.arena_balls(14, radius=3, arena=30, gap=0.0, steps=0, seed=5)
+    m.init_velocity = -20.0 * m.voxel_size * (m.ijk - m.ijk.mean(0))   # towards each other
+    nl = len(engine.topology(m)[0])
+    c = engine.Batch(precision=precision, path=_abi.PATH_STREAM, collision_rebuild_interval=5)
+    r = c.admit(m)
+    c.step_noalloc(30)
+    b = engine.Batch(precision=precision, path=_abi.PATH_STREAM, collision_rebuild_interval=5,
+                     collision_table_entries=2 * len(c.collision_pairs(r)) + 1)
+    s = b.admit(m)
+    done, stood = 0, 0
+    c.retire(r)
+    r = c.admit(m)
+    for _ in range(40):
+        b.step(7)
+        got = b.read_state(s, nl=nl)
+        try:
+            pairs = b.collision_pairs(s)
+        except engine.VX3Error:
+            pairs = None
+        steps = b.poll()[s].steps
+        if steps > done:
+            c.step_noalloc(steps - done)
+        ref = c.read_state(r, nl=nl)
+        for k in KEYS:
+            assert np.array_equal(got[k], ref[k]), (k, steps)
+        if steps < done + 7:
+            assert pairs is None
+            with pytest.raises(engine.VX3Error):   # not before the next step either
+                b.collision_pairs(s)
+            stood += steps > 0
+        else:
+            assert np.array_equal(pairs, c.collision_pairs(r))
+        done = steps
+    assert stood > 0 and done > 200
+    b.close()
+    c.close()
