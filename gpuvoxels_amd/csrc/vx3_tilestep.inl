@@ -94,8 +94,9 @@ template <typename E> __device__ __forceinline__ E& lrow(char* rec, int off, uns
 // reports are agent-scope stores: every tile that writes one writes the same value
 __device__ __forceinline__ void tsSay(unsigned* word, unsigned seq) { __hip_atomic_store(word, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// A float no smaller than |x| of a displacement x^2 = d2
-__device__ __forceinline__ float tsReach(real d2) { return sqrtf((float)d2 * (1.0f + 0x1p-20f)) * (1.0f + 0x1p-20f); }
+// A float no smaller than |x| of a displacement x^2 = d2; of a NaN none (such a voxel is nobody's
+// partner, and must not make its tile's bounds NaN)
+__device__ __forceinline__ float tsReach(real d2) { return d2 >= 0 ? sqrtf((float)d2 * (1.0f + 0x1p-20f)) * (1.0f + 0x1p-20f) : 0.0f; }
 
 // Bounds of the workgroup's surface voxels (mine: this thread's is one) into hull and box of
 // parity p, and each wave's into red; empty where there are none.  All widened by *widen (LDS;
@@ -416,7 +417,7 @@ __device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& t
         const int w = tid / 6, a = tid % 3;
         const float r = sqrtf(sc.colThreshSq) * (1.0f + 0x1p-20f);
         const float l = sReach[w][a], h = sReach[w][3 + a];
-        const float e = r + (fmaxf(fabsf(l), fabsf(h)) + r) * 0x1p-20f;
+        const float e = l <= h ? r + (fmaxf(fabsf(l), fabsf(h)) + r) * 0x1p-20f : 0.0f;
         sWide[w][tid % 6] = tid % 6 < 3 ? l - e : h + e;   // (of no voxels: stays empty, +inf and -inf)
     }
     __syncthreads();
@@ -457,7 +458,7 @@ __device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& t
                 for (int q = 0; q < 4; q++) {
                     const int k = 32 * half + i + q;
                     const real dx = x - lanes(cx, k), dy = y - lanes(cy, k), dz = z - lanes(cz, k);
-                    w = w + w + (unsigned)!(dx * dx + dy * dy + dz * dz > thresh);
+                    w = w + w + (unsigned)(dx * dx + dy * dy + dz * dz <= thresh);   // (a NaN is near nothing)
                 }
             near[half] = mine ? (w << (32 - i)) & (0xFFFFFFFFu << (32 - left)) : 0u;
         }
@@ -529,7 +530,8 @@ __device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& t
         if (tid == 0) sN = 0;
         before = 0;
         constexpr int W = VX3_TS_BLOCK / 64, AT_ONCE = 4;
-        // another tile's bounds are of its last rebuild: widened by how far its voxels moved
+        // another tile's bounds are of its last rebuild: widened by how far its voxels moved (of no
+        // voxels, +inf and -inf: NaN, which meets nothing)
         auto wider = [](float* e, float m) {
 #pragma unroll
             for (int k = 0; k < 6; k++) {

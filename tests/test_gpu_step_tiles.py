@@ -189,3 +189,15 @@ def test_standing_still_for_a_table_changes_nothing(precision):
     assert stood > 0 and done > 200
     b.close()
     c.close()
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_bodies_beside_one_that_is_lost(precision, bad):
+    """One voxel thrown with a velocity that is no number: its body is lost, the lists and the
+    motion of the others, some of them in its tile, are those of the per-step kernels."""
+    m = workloads.arena_balls(90, radius=1, arena=18, gap=0.0, sigma_v=0.4, steps=0, seed=5)
+    m.init_velocity[100, 1] = bad
+    a, c = (run([m], [60, 60], k, precision, 8) for k in (False, True))
+    assert np.isnan(c[0][0]["pos"]).any() and not np.isnan(c[0][0]["pos"]).all() and len(c[0][1]) > 0
+    assert_equal(a, c)
