@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdarg>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -206,6 +207,8 @@ struct vx3h_batch {
     // at least VX3_TS_MIN_STEPS steps
     std::vector<int> stepSims;                   // slots, in admission order
     bool stepDirty = false;
+    std::atomic<long long> stepVoxels{0};        // theirs (read by the threads that prepare admissions)
+    long long stepTileCount = 0;
     TsTile* dStepTiles = nullptr; size_t capStepTiles = 0;
     int nStepTiles = 0;
     int stepShape = 0;
@@ -948,6 +951,9 @@ vx3h_status syncStep(vx3h_batch* b) {
     return VX3H_OK;
 }
 
+// whether the simulations with step tiles take long calls on the fused kernel
+bool fusedSteps(const vx3h_batch* b) { return !b->stepSims.empty() && stepTilesPay(b->stepTileCount, b->stepVoxels.load(), b->realSize); }
+
 // n launches of the fused kernel (what: TS_LOAD and TS_STORE once, around a call's steps; the
 // load's n: the steps of the call)
 vx3h_status launchStepTiles(vx3h_batch* b, int what, int n) {
@@ -1246,10 +1252,11 @@ struct PreparedSim {
     StepTilePlan stepPlan;
 };
 
-bool stepPlanOf(const HostModel& H, StepTilePlan* out) {
+bool stepPlanOf(const vx3h_batch* b, const HostModel& H, StepTilePlan* out) {
     std::vector<char> interior(H.nv);
     for (int v = 0; v < H.nv; v++) interior[v] = (H.vflags[v] & VF_INTERIOR) != 0;
-    return planStepTiles(H.nv, H.ijk.data(), H.nl, H.lneg.data(), H.lpos.data(), H.voxelLinks.data(), interior.data(), out);
+    return planStepTiles(H.nv, H.ijk.data(), H.nl, H.lneg.data(), H.lpos.data(), H.voxelLinks.data(), interior.data(), out,
+                         b->stepVoxels.load(std::memory_order_relaxed));
 }
 
 // the tile plan a simulation of this model gets if it is too large for one workgroup
@@ -1282,7 +1289,7 @@ vx3h_status prepareSim(const vx3h_batch* b, const vx3h_sim_desc* desc, PreparedS
         for (int i = 0; i < H.nl; i++) perAxis[H.laxis[i]]++;
         const int lax = r.block * r.lpa;
         if (H.nv > r.block * r.vpt || perAxis[0] > lax || perAxis[1] > lax || perAxis[2] > lax)
-            p->stepPlanned = stepPlanOf(H, &p->stepPlan);
+            p->stepPlanned = stepPlanOf(b, H, &p->stepPlan);
     }
     *out = p;
     return VX3H_OK;
@@ -1543,8 +1550,9 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     bool stepped = shape < 0 && !tiles && NV > 0 && resOk && b->cfg.path != VX3H_PATH_RESIDENT;
     if (stepped) {
         if (pre && pre->stepPlanned) splan = std::move(pre->stepPlan);
-        else stepped = stepPlanOf(H, &splan);
+        else stepped = stepPlanOf(b, H, &splan);
     }
+    if (stepped) stepped = stepTilesPay((long long)splan.tiles.size(), NV, rs);
     if (stepped) {
         size_t freeB = 0, totB = 0;
         HIPCHK(hipMemGetInfo(&freeB, &totB));
@@ -1781,6 +1789,8 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     } else if (stepped) {
         if (vx3h_status st = placeStep(b, sh, H, splan)) return st;
         b->stepSims.push_back(s);
+        b->stepVoxels += NV;
+        b->stepTileCount += (long long)sh.stepTiles.size();
         b->stepDirty = true;
     }
     else b->nStreamSims++;
@@ -1847,7 +1857,7 @@ extern "C" vx3h_status vx3h_batch_step(vx3h_batch* b, int n_steps) {
     // and so does the first step of a simulation that stood still after its link pass.
     const bool resume = b->resumePending;
     b->resumePending = false;   // every waiting simulation resumes in the first step below
-    const bool fused = !b->stepSims.empty() && n_steps >= VX3_TS_MIN_STEPS;
+    const bool fused = n_steps >= VX3_TS_MIN_STEPS && fusedSteps(b);
     if (fused)
         if (vx3h_status st = syncStep(b)) return st;
     bool loaded = false;
@@ -2069,16 +2079,19 @@ extern "C" vx3h_status vx3h_batch_kernel_times(vx3h_batch* b, int n_steps, doubl
     std::vector<hipEvent_t> ev(2 * PASS_COUNT * n_steps, nullptr);
     for (auto& e : ev) HIPCHK(hipEventCreate(&e));
     const StepOpts o = stepOpts(b);
+    const bool fused = fusedSteps(b);
+    DevBatch<float> view = b->db;
+    view.solo = fused ? -1 : -3;
     for (int i = 0; i < n_steps; i++) {
         hipEvent_t* e = &ev[2 * PASS_COUNT * i];
-        if (b->realSize == 4) launchStep(b->db, b->stream, o, e);
-        else launchStep(*reinterpret_cast<DevBatch<double>*>(&b->db), b->stream, o, e);
+        if (b->realSize == 4) launchStep(view, b->stream, o, e);
+        else launchStep(*reinterpret_cast<DevBatch<double>*>(&view), b->stream, o, e);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(b->stream));
     const bool ran[PASS_COUNT] = {false, b->db.lHi > 0, o.contacts, true, true};   // Poisson: part of the voxel pass
     for (int k = 0; k < PASS_COUNT; k++) {
-        if (!ran[k] || b->nStreamSims == 0) continue;
+        if (!ran[k] || (b->nStreamSims == 0 && (fused || b->stepSims.empty()))) continue;
         double tot = 0;
         for (int i = 0; i < n_steps; i++) {
             float ms = 0;
@@ -2107,7 +2120,7 @@ extern "C" vx3h_status vx3h_batch_kernel_times(vx3h_batch* b, int n_steps, doubl
         avg_ms[5] += ms;
     }
     for (auto& e : rev) hipEventDestroy(e);
-    if (!b->stepSims.empty()) {   // the fused per-step kernel: the steps' summed duration
+    if (fused) {   // the fused per-step kernel: the steps' summed duration
         if ((st = syncStep(b))) return st;
         hipEvent_t e0, e1;
         HIPCHK(hipEventCreate(&e0));
@@ -2470,6 +2483,8 @@ extern "C" vx3h_status vx3h_sim_retire(vx3h_batch* b, int slot) {
         b->tileDirty = true;
     } else if (!sh.stepTiles.empty()) {
         b->stepSims.erase(std::remove(b->stepSims.begin(), b->stepSims.end(), slot), b->stepSims.end());
+        b->stepVoxels -= sh.nv;
+        b->stepTileCount -= (long long)sh.stepTiles.size();
         releaseStep(b, sh);
         b->stepDirty = b->tileDirty = true;
     } else { b->nStreamSims--; b->tileDirty = true; }

@@ -100,7 +100,7 @@ uint64_t spread(uint64_t x) {   // 21 bits to every third bit
 }  // namespace
 
 bool planStepTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos, const int* vlinks,
-                   const char* interior, StepTilePlan* out) {
+                   const char* interior, StepTilePlan* out, long long beside) {
     *out = StepTilePlan();
     if (nv <= 0) return false;
     int low[3];
@@ -176,7 +176,14 @@ bool planStepTiles(int nv, const int* ijk, int nl, const int* lneg, const int* l
     //   per-step kernels         58.8      -   66.7            132.2         64.8
     // close: the box around them, a margin of 2 included, has less than 2.25 times their boxes'
     // volume (1.3 and 1.7 times: up to half as slow again, 3 times: no faster).
-    const size_t fill = std::max(64, std::min(VX3_TS_BLOCK, (nv + 383) / 384));
+    // Many simulations side by side share the units: a tile is also filled to 1/640 of all their
+    // voxels.  us per step, by the simulation's own alone and by both, FP64 and FP32 (from 1/384 to
+    // 1/512 of all, 20 of 60 cubes of 4^3 are 8 to 12% slower, else it is the same):
+    //   60 simulations of 120 cubes of 3^3     169.3  127.0    128.9   96.2
+    //   30 of 100 balls of radius 2             79.4   66.7     75.0   71.8
+    //   30 of 300 balls of radius 3            306.9  256.1    266.7  200.0
+    const long long share = std::max((nv + 383LL) / 384, (nv + beside + 639) / 640);
+    const size_t fill = (size_t)std::max(64LL, std::min((long long)VX3_TS_BLOCK, share));
     std::vector<int> open, body(nv, 0);   // (body: of the small ones, in that order)
     long long volumes = 0;   // of the boxes of those in `open`, and the box around them
     int box[2][3] = {};

@@ -23,10 +23,27 @@ struct StepTilePlan {
 
 // Cuts the voxels [0, nv) (lattice indices ijk; vlinks: six link indices per voxel, -1 =
 // none; interior per voxel) joined by links into tiles: connected bodies that fit a tile
-// stay whole, near ones together where they are many and small; larger ones are cut into compact lattice blocks.  False
+// stay whole, near ones together where they are many and small; larger ones are cut into compact lattice blocks.
+// beside: voxels that other simulations step beside these in the same launches.  False
 // for an empty simulation or a lattice of more than 2^16 along an axis.
 bool planStepTiles(int nv, const int* ijk, int nl, const int* lneg, const int* lpos, const int* vlinks,
-                   const char* interior, StepTilePlan* out);
+                   const char* interior, StepTilePlan* out, long long beside = 0);
+
+// Whether a launch of `tiles` tiles with `voxels` voxels in them steps faster than the per-step
+// kernels, whose time follows the voxels, not the tiles: small bodies that are far apart hardly
+// share tiles.  Measured on MI355X, us per step, lists rebuilt every 8 steps, per-step kernels
+// and fused, FP64 and FP32:
+//                                      tiles   voxels         FP64           FP32
+//   2,000 lone voxels, 8 apart           979    2,000    24.2   20.1    23.0   20.2
+//   4,000                              2,000    4,000    24.7   31.4    23.1   32.0
+//   2,000 cubes of 2^3, 12 apart         865   16,000    41.8   37.2    38.3   34.6
+//   4,000                              1,740   32,000    47.9   55.2    41.5   51.0
+//   4,000 cubes of 3^3, 20 apart       1,876  108,000    88.7   66.5    72.2   61.4
+//   8,000 balls of 33, 16 apart        3,980  264,000   139.4  130.4   105.8  118.5
+//   8,000 cubes of 4^3, 24 apart       4,494  512,000   310.9  163.5   216.7  139.1
+inline bool stepTilesPay(long long tiles, long long voxels, size_t realBytes) {
+    return tiles <= 1000 || voxels >= (realBytes == 8 ? 80 : 96) * (tiles - 1000);
+}
 
 // The numbers under which the fused kernel's steps report (TsReport).  Report words are matched
 // by number and never cleared one by one, so a number is used once: when a call's would pass the

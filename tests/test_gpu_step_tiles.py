@@ -201,3 +201,34 @@ def test_bodies_beside_one_that_is_lost(precision, bad):
     a, c = (run([m], [60, 60], k, precision, 8) for k in (False, True))
     assert np.isnan(c[0][0]["pos"]).any() and not np.isnan(c[0][0]["pos"]).all() and len(c[0][1]) > 0
     assert_equal(a, c)
+
+
+def test_bodies_too_sparse_for_tiles():
+    """Lone voxels far apart: one simulation's on the fused kernel, two simulations' on the per-step
+    kernels, and back after one has left; each as on the per-step kernels throughout."""
+    def lone(seed):
+        m = workloads.arena_balls(2, radius=1, arena=20, steps=0)
+        g = np.stack(np.meshgrid(np.arange(40), np.arange(30), indexing="ij"), -1).reshape(-1, 2) * 8
+        m.ijk = np.concatenate([g, np.zeros((len(g), 1), int)], 1).astype(np.int32)
+        m.ijk = m.ijk[np.lexsort((m.ijk[:, 0], m.ijk[:, 1]))]
+        m.mat, m.phase = np.zeros(len(g), np.int32), None
+        m.init_velocity = np.random.default_rng(seed).normal(0, 0.5, (len(g), 3))
+        return m
+    models = [lone(1), lone(2), lone(3)]
+    got = []
+    for noalloc in (False, True):
+        b = engine.Batch(precision=_abi.PREC_F64, path=_abi.PATH_STREAM, collision_rebuild_interval=8)
+        step = b.step_noalloc if noalloc else b.step
+        s = [b.admit(models[0])]
+        step(30)
+        s.append(b.admit(models[1]))
+        step(30)
+        b.retire(s[0])
+        step(30)
+        s[0] = b.admit(models[2])
+        step(30)
+        got.append([b.read_state(x) for x in s])
+        b.close()
+    for x, y in zip(*got):
+        for k in ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac"):
+            assert np.array_equal(x[k], y[k]), k
