@@ -413,6 +413,8 @@ __device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& t
     // more than the boxes' float rounding (2^-24 of each coordinate) can explain, so that no
     // watched pair is missed
     tsBox(ts.aux[td.rec], 1 - ts.par, mine, (float)x, (float)y, (float)z, sReach, nullptr);
+    // inside a body: no lists (FP32 cube of 192^3, rebuilt every 8 steps: 2,207 -> 1,731 us a step)
+    if (td.nSurf == 0) return true;
     if (tid < VX3_TS_BLOCK / 64 * 6) {
         const int w = tid / 6, a = tid % 3;
         const float r = sqrtf(sc.colThreshSq) * (1.0f + 0x1p-20f);

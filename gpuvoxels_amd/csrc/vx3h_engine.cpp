@@ -1552,7 +1552,11 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
         if (pre && pre->stepPlanned) splan = std::move(pre->stepPlan);
         else stepped = stepPlanOf(b, H, &splan);
     }
-    if (stepped) stepped = stepTilesPay((long long)splan.tiles.size(), NV, rs);
+    if (stepped) {
+        const long long T = (long long)splan.tiles.size();
+        const auto surface = std::count_if(splan.tiles.begin(), splan.tiles.end(), [](const TsTile& t) { return t.nSurf > 0; });
+        stepped = stepTilesPay(T, NV, rs) && (!H.collisions || stepRebuildsPay(T, surface));
+    }
     if (stepped) {
         size_t freeB = 0, totB = 0;
         HIPCHK(hipMemGetInfo(&freeB, &totB));

@@ -45,6 +45,13 @@ inline bool stepTilesPay(long long tiles, long long voxels, size_t realBytes) {
     return tiles <= 1000 || voxels >= (realBytes == 8 ? 80 : 96) * (tiles - 1000);
 }
 
+// Whether the fused kernel's list rebuilds pay too: each tile with surface voxels (`surface` of a
+// simulation's `tiles`) reads the bounds of all, where the per-step kernels hash the voxels.
+// Measured on MI355X, us per step, balls of 257 voxels in FP32, one a tile, rebuilt every 8 steps,
+// per-step kernels and fused: 16,384 balls 1,727 and 1,074, 32,768 balls 3,556 and 2,338, 65,536
+// balls 7,193 and 6,475.
+inline bool stepRebuildsPay(long long tiles, long long surface) { return surface <= (1LL << 32) / (tiles > 0 ? tiles : 1); }
+
 // The numbers under which the fused kernel's steps report (TsReport).  Report words are matched
 // by number and never cleared one by one, so a number is used once: when a call's would pass the
 // largest, all words have to be cleared and the numbers start over.

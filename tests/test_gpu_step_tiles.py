@@ -232,3 +232,12 @@ def test_bodies_too_sparse_for_tiles():
     for x, y in zip(*got):
         for k in ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac"):
             assert np.array_equal(x[k], y[k]), k
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+def test_tiles_without_surface(precision):
+    """A body thick enough for tiles inside it that have no surface voxel, touched from above."""
+    m = workloads.drop(26, gap=1, shift=3, steps=0)
+    a, c = (run([m], [9, 40], k, precision, 8) for k in (False, True))
+    assert len(a[0][1]) > 0
+    assert_equal(a, c)

@@ -51,3 +51,15 @@ def test_when_tiles_pay(tmp_path):
     lines = "\n".join("%d %d %d" % c for c in faster + slower)
     out = subprocess.run([exe], input=lines, stdout=subprocess.PIPE, text=True, check=True).stdout
     assert out == "1" * len(faster) + "0" * len(slower)
+
+
+def test_when_rebuilds_pay(tmp_path):
+    src = tmp_path / "pay.cpp"
+    src.write_text('#include <cstdio>\n#include "%s"\nint main() {\n    long long t, s;\n'
+                   '    while (scanf("%%lld %%lld", &t, &s) == 2) printf("%%d", (int)vx3::stepRebuildsPay(t, s));\n}\n'
+                   % os.path.join(CSRC, "vx3h_steptile.h"))
+    exe = str(tmp_path / "pay")
+    subprocess.run(["g++", "-std=c++17", "-o", exe, str(src)], check=True)
+    out = subprocess.run([exe], input="1 1\n65536 65536\n36864 6500\n131072 131072\n4194303 4194303\n4194303 100\n",
+                         stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert out == "111001"
