@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstddef>
 #include <cstdio>
 #include <cstdarg>
 #include <array>
@@ -351,6 +352,9 @@ vx3h_status fillBytes(vx3h_batch* b, void* dst, int value, size_t bytes) {
     return VX3H_OK;
 }
 
+size_t stepBytes(const vx3h_batch* b);
+vx3h_status dropStepTiles(vx3h_batch* b);
+
 vx3h_status growArrays(vx3h_batch* b, std::vector<ArrSpec>& arrs, int& cap, int need, int used, bool isVoxel) {
     if (need <= cap) return VX3H_OK;
     int ncap = std::max(need, std::max(2 * cap, 1024));
@@ -365,6 +369,10 @@ vx3h_status growArrays(vx3h_batch* b, std::vector<ArrSpec>& arrs, int& cap, int 
             largest = std::max(largest, (size_t)ncap * a.per * a.elem);
         }
         HIPCHK(hipMemGetInfo(&freeB, &totalB));
+        if (grow + largest > freeB && stepBytes(b) > 0) {
+            if (vx3h_status st = dropStepTiles(b)) return st;
+            HIPCHK(hipMemGetInfo(&freeB, &totalB));
+        }
         if (grow + largest > freeB) FAILV(VX3H_ENOMEM, "device memory too small to grow the batch arrays");
     }
     for (ArrSpec& a : arrs) {
@@ -413,8 +421,14 @@ vx3h_status poolGrow(vx3h_batch* b, DevPool& p) {
     return VX3H_OK;
 }
 
+// (The batch is between calls: without device memory the fused kernel's copies make room.)
 vx3h_status poolAlloc(vx3h_batch* b, DevPool& p, int n, int& start) {
-    return takeRange(p, n, start, [&](DevPool& q) { return poolGrow(b, q); });
+    auto grow = [&](DevPool& q) { return poolGrow(b, q); };
+    const vx3h_status st = takeRange(p, n, start, grow);
+    if (st != VX3H_EDEVICE || stepBytes(b) == 0) return st;
+    (void)hipGetLastError();
+    if (vx3h_status ds = dropStepTiles(b)) return ds;
+    return takeRange(p, n, start, grow);
 }
 
 template <typename E> vx3h_status uploadTable(vx3h_batch* b, void*& dptr, size_t& cap, const std::vector<E>& v) {
@@ -833,19 +847,31 @@ vx3h_status stepCtl(vx3h_batch* b) {
     return VX3H_OK;
 }
 
-// device memory a plan's growth of the pools needs (old and new arrays exist side by side
-// while one is replaced)
-size_t stepGrowth(const vx3h_batch* b, const StepTilePlan& p, int nv) {
+// device memory that the fused kernel's pools hold
+size_t stepBytes(const vx3h_batch* b) {
+    size_t tot = (size_t)b->stepCtlCap * 2 * (sizeof(TsCtl) + sizeof(TsReport));
+    for (const DevPool* q : {&b->stepTilePool, &b->stepPhasePool, &b->stepO2pPool, &b->stepCtlPool})
+        for (const auto& a : q->arrs) tot += (size_t)q->cap * a.second;
+    return tot;
+}
+
+// What a plan's growth of the pools allocates (old and new arrays exist side by side while one
+// is replaced); *held: what the pools hold in the end.
+size_t stepGrowth(const vx3h_batch* b, const StepTilePlan& p, int nv, size_t* held) {
     size_t tot = 0;
-    auto grow = [&](const DevPool& q, size_t n) {
+    *held = stepBytes(b);
+    auto grow = [&](const DevPool& q, size_t n, size_t beside) {
         if ((size_t)q.ra.hi + n <= (size_t)q.cap) return;
         const size_t c = std::max((size_t)q.ra.hi + n, (size_t)std::max(2 * q.cap, q.minCap));
-        for (const auto& a : q.arrs) tot += c * a.second;
+        size_t each = beside;
+        for (const auto& a : q.arrs) each += a.second;
+        tot += c * each;
+        *held += (c - (size_t)q.cap) * each;
     };
-    grow(b->stepTilePool, p.tiles.size());
-    grow(b->stepPhasePool, RES_MAX_PHASES);
-    grow(b->stepO2pPool, nv);
-    grow(b->stepCtlPool, 1);
+    grow(b->stepTilePool, p.tiles.size(), 0);
+    grow(b->stepPhasePool, RES_MAX_PHASES, 0);
+    grow(b->stepO2pPool, nv, 0);
+    grow(b->stepCtlPool, 1, 2 * (sizeof(TsCtl) + sizeof(TsReport)));
     return tot;
 }
 
@@ -857,7 +883,44 @@ void releaseStep(vx3h_batch* b, SlotHost& sh) {
     sh.stepTiles.clear();
 }
 
-// A simulation's step tiles: ranges in the pools, tables uploaded.  sh.v0, l0 and nv are set.
+// Gives the fused kernel's device memory back, between calls (the state is in the batch arrays):
+// its simulations step on the per-step kernels from then on.
+vx3h_status dropStepTiles(vx3h_batch* b) {
+    HIPCHK(hipStreamSynchronize(b->stream));
+    for (int s : b->stepSims) {
+        int* const at = (int*)((char*)(b->db.sims + s) + offsetof(SimCtl, flags));
+        int flags;
+        HIPCHK(hipMemcpy(&flags, at, sizeof(int), hipMemcpyDeviceToHost));
+        flags &= ~SC_TILESTEP;
+        HIPCHK(hipMemcpy(at, &flags, sizeof(int), hipMemcpyHostToDevice));
+    }
+    b->nStreamSims += (int)b->stepSims.size();
+    for (int s : b->stepSims) b->slots[s].stepTiles.clear();
+    b->stepSims.clear();
+    b->stepVoxels = 0;
+    b->stepTileCount = 0;
+    b->nStepTiles = 0;
+    b->stepDirty = b->tileDirty = true;
+    b->layout++;
+    TsArgs& t = b->ts;
+    for (DevPool* q : {&b->stepTilePool, &b->stepPhasePool, &b->stepO2pPool, &b->stepCtlPool}) {
+        for (auto& a : q->arrs) {
+            if (*a.first) HIPCHK(hipFree(*a.first));
+            *a.first = nullptr;
+        }
+        q->cap = 0;
+        q->ra = RangeAlloc();
+    }
+    if (t.ctl) HIPCHK(hipFree(t.ctl));
+    t.ctl = nullptr;
+    if (t.report) HIPCHK(hipFree(t.report));
+    t.report = nullptr;
+    b->stepCtlCap = t.ctlCap = 0;
+    return VX3H_OK;
+}
+
+// A simulation's step tiles: ranges in the pools, tables uploaded; after an error it has none.
+// sh.v0, l0 and nv are set.
 vx3h_status placeStep(vx3h_batch* b, SlotHost& sh, const HostModel& H, StepTilePlan& p) {
     const int T = (int)p.tiles.size();
     std::vector<double> phases;
@@ -879,11 +942,17 @@ vx3h_status placeStep(vx3h_batch* b, SlotHost& sh, const HostModel& H, StepTileP
         }
     }
     sh.tqN = (int)phases.size();
-    vx3h_status e;
-    if ((e = poolAlloc(b, b->stepTilePool, T, sh.ts0)) || (e = poolAlloc(b, b->stepPhasePool, sh.tqN, sh.tq0)) ||
-        (e = poolAlloc(b, b->stepO2pPool, H.nv, sh.to0)) || (e = poolAlloc(b, b->stepCtlPool, 1, sh.tc0)) || (e = stepCtl(b)))
-        return e;
-    if (b->stepTilePool.ra.hi > (INT32_MAX >> VX3_TS_SLOT_BITS)) FAILV(VX3H_ENOMEM, "too many step tiles");
+    DevPool* const pools[4] = {&b->stepTilePool, &b->stepPhasePool, &b->stepO2pPool, &b->stepCtlPool};
+    const int need[4] = {T, sh.tqN, H.nv, 1};
+    int* const start[4] = {&sh.ts0, &sh.tq0, &sh.to0, &sh.tc0};
+    vx3h_status e = takeRanges(pools, need, start, [&](DevPool& q) { return poolGrow(b, q); });
+    if (e) return e;
+    sh.stepTiles = p.tiles;
+    sh.maxStepSlots = p.maxSlots;
+    sh.maxStepOwn = p.maxOwn;
+    auto undo = [&](vx3h_status st) { releaseStep(b, sh); return st; };
+    if ((e = stepCtl(b))) return undo(e);
+    if (b->stepTilePool.ra.hi > (INT32_MAX >> VX3_TS_SLOT_BITS)) return undo(VX3H_ENOMEM);
     std::vector<char> tab(VX3_TS_TAB, 0);   // by the simulation's own material indices
     memcpy(tab.data(), H.vmats.data(), H.vmats.size() * sizeof(VoxMatDev));
     memcpy(tab.data() + RES_MAX_VMATS * sizeof(VoxMatDev), H.lmats.data(), H.lmats.size() * sizeof(LinkMatDev));
@@ -907,16 +976,14 @@ vx3h_status placeStep(vx3h_batch* b, SlotHost& sh, const HostModel& H, StepTileP
     }
     const TsArgs& t = b->ts;
     char* stage;   // the records' first part, one strided copy
-    if ((e = stageAlloc(b, p.stat.size(), &stage))) return e;
+    if ((e = stageAlloc(b, p.stat.size(), &stage))) return undo(e);
     memcpy(stage, p.stat.data(), p.stat.size());
-    HIPCHK(hipMemcpy2DAsync(t.stat + (size_t)sh.ts0 * TsStat::BYTES, TsStat::BYTES, stage, TsStat::ST_END, TsStat::ST_END, T,
-                            hipMemcpyHostToDevice, b->stream));
+    if (hipMemcpy2DAsync(t.stat + (size_t)sh.ts0 * TsStat::BYTES, TsStat::BYTES, stage, TsStat::ST_END, TsStat::ST_END, T,
+                         hipMemcpyHostToDevice, b->stream) != hipSuccess)
+        return undo(VX3H_EDEVICE);
     if ((e = upload(b, (char*)t.tab + (size_t)sh.tc0 * VX3_TS_TAB, tab.data(), tab.size())) ||
         (e = upload(b, (void*)(t.ph + sh.tq0), phases.data(), phases.size() * 8)) || (e = upload(b, (void*)(t.o2p + sh.to0), o2p.data(), o2p.size() * 4)))
-        return e;
-    sh.stepTiles = p.tiles;
-    sh.maxStepSlots = p.maxSlots;
-    sh.maxStepOwn = p.maxOwn;
+        return undo(e);
     return VX3H_OK;
 }
 
@@ -1345,6 +1412,8 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     if (b->bytesUsed + need > b->budget) FAILV(VX3H_ENOMEM, "simulation does not fit the batch's device memory budget");
     HIPCHK(hipStreamSynchronize(b->stream));
     b->stageUsed = 0;   // the stream has run every staged copy
+    if (b->bytesUsed + need + stepBytes(b) > b->budget)   // the fused kernel's copies take only what is left of the budget
+        if (vx3h_status st = dropStepTiles(b)) return st;
     // slot
     int s = -1;
     for (int i = 0; i < (int)b->slots.size(); i++) if (!b->slots[i].used) { s = i; break; }
@@ -1544,8 +1613,8 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
         FAILV(VX3H_EUNSUPPORTED,
               "detach, attach, secondary experiments, signals, target contacts and close pairs run on the stream path");
     // too large for the resident kernels, without topology changes or extra forces: the
-    // fused per-step kernel, where the device memory that later admissions may still claim
-    // (the rest of the budget) leaves room for its tile arrays
+    // fused per-step kernel, where the budget leaves room for its copies of the state (a later
+    // admission that needs the room gets it, see dropStepTiles)
     StepTilePlan splan;
     bool stepped = shape < 0 && !tiles && NV > 0 && resOk && b->cfg.path != VX3H_PATH_RESIDENT;
     if (stepped) {
@@ -1560,9 +1629,10 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     if (stepped) {
         size_t freeB = 0, totB = 0;
         HIPCHK(hipMemGetInfo(&freeB, &totB));
-        const size_t later = b->budget > b->bytesUsed + need ? b->budget - b->bytesUsed - need : 0;
-        const size_t grow = stepGrowth(b, splan, NV);
-        if (grow > 0 && freeB < later + grow) stepped = false;
+        size_t held;
+        const size_t grow = stepGrowth(b, splan, NV, &held);
+        // (and a sixteenth of the budget stays free for what is not counted)
+        stepped = b->bytesUsed + need + held <= b->budget && (grow == 0 || grow + b->budget / 16 <= freeB);
     }
     // control block
     SimCtl c;
@@ -1790,14 +1860,20 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
         b->resLists[sh.shape].push_back(s);
         b->resDirty = true;
         b->tileDirty = true;
-    } else if (stepped) {
-        if (vx3h_status st = placeStep(b, sh, H, splan)) return st;
+    } else if (stepped && placeStep(b, sh, H, splan) == VX3H_OK) {
         b->stepSims.push_back(s);
         b->stepVoxels += NV;
         b->stepTileCount += (long long)sh.stepTiles.size();
         b->stepDirty = true;
     }
-    else b->nStreamSims++;
+    else {
+        if (stepped) {   // no room for its step tiles after all
+            (void)hipGetLastError();
+            c.flags &= ~SC_TILESTEP;
+            UPLOAD(b->db.sims + s, &c, sizeof(c));
+        }
+        b->nStreamSims++;
+    }
     if (!tiles && shape < 0) b->tileDirty = true;   // which tiles run depends on what else does
     sh.vlinks = H.voxelLinks;
     sh.surface.resize(NV);
@@ -2398,6 +2474,7 @@ vx3h_status growCollisionTables(vx3h_batch* b, std::vector<SimCtl>& ctl) {
         c.nearUsed = 0;
         if (c.flags & SC_LINKS_DONE) b->resumePending = true;
         c.flags = (c.flags & ~SC_COL_GROW) | SC_REBUILD;
+        if (sh.stepTiles.empty()) c.flags &= ~SC_TILESTEP;   // (given up above, for the table)
         HIPCHK(hipMemcpy(b->db.sims + s, &c, sizeof(SimCtl), hipMemcpyHostToDevice));
         b->db.Ccap = b->nbPool.cap;
         b->tableGrowths++;

@@ -276,7 +276,9 @@ enum {
 enum { VX3H_PREC_F32 = 0, VX3H_PREC_F64 = 1 };
 
 typedef struct vx3h_batch_cfg {
-    size_t max_device_bytes;  /* admission budget for simulation state; 0 = 90% of free HBM */
+    size_t max_device_bytes;  /* admission budget for simulation state; 0 = 90% of free HBM.  The fused
+                                 per-step kernel's copies of the state (about as much again) take what
+                                 it leaves, and are given up when an admission needs the room */
     int    precision;         /* VX3H_PREC_*: F64 state meets the reference's trajectories over the
                                  full horizon; F32 state is faster and meets them over short horizons */
     int    path;              /* VX3H_PATH_* */

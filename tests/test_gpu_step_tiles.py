@@ -241,3 +241,52 @@ def test_tiles_without_surface(precision):
     a, c = (run([m], [9, 40], k, precision, 8) for k in (False, True))
     assert len(a[0][1]) > 0
     assert_equal(a, c)
+
+
+def test_tiles_stay_within_the_budget():
+    """The fused kernel's copies of the state take what the batch's device memory budget leaves:
+    not used where it leaves too little, given up when a later admission needs the room; the
+    same results throughout."""
+    first, second = workloads.drop(12, gap=1, shift=3, steps=0), workloads.drop(11, gap=1, shift=2, steps=0)
+    import ctypes as C
+    need = []
+    for m in (first, second):
+        n = C.c_size_t(0)
+        desc, keep = m.desc()
+        engine.check(engine.lib().vx3h_sim_footprint(C.byref(desc), _abi.PREC_F64, C.byref(n)))
+        need.append(n.value)
+    fused = lambda b: "voxels" not in b.kernel_times(4)  # noqa: E731
+    b = engine.Batch(precision=_abi.PREC_F64, path=_abi.PATH_STREAM, max_device_bytes=need[0] + 100000)
+    b.admit(first)
+    b.step(8)
+    assert not fused(b)
+    b.close()
+    tiles = 64 * 270000   # room for the tiles of the first, not for those of both
+    got = []
+    for noalloc in (False, True):
+        b = engine.Batch(precision=_abi.PREC_F64, path=_abi.PATH_STREAM, max_device_bytes=need[0] + tiles)
+        step = b.step_noalloc if noalloc else b.step
+        s = b.admit(first)
+        step(40)
+        if not noalloc:
+            assert fused(b)
+        else:
+            step(4)
+        b.retire(b.admit(workloads.cube(3, steps=0)))
+        t = []
+        while True:   # until the budget holds no more
+            try:
+                t.append(b.admit(second))
+            except engine.VX3Error:
+                break
+        assert len(t) == tiles // need[1]
+        step(40)
+        if not noalloc:
+            assert not fused(b)
+        else:
+            step(4)
+        got.append([b.read_state(x) for x in [s] + t])
+        b.close()
+    for x, y in zip(*got):
+        for k in ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac"):
+            assert np.array_equal(x[k], y[k]), k
