@@ -290,3 +290,32 @@ def test_tiles_stay_within_the_budget():
     for x, y in zip(*got):
         for k in ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac"):
             assert np.array_equal(x[k], y[k]), k
+
+
+@pytest.mark.parametrize("precision,graph", [(_abi.PREC_F64, 1), (_abi.PREC_F32, 1), (_abi.PREC_F64, 0)])
+def test_beside_the_per_step_kernels(precision, graph):
+    """Fused simulations beside one that only the per-step kernels take, and a one-workgroup one:
+    calls of several chunks and short ones in between; the bits of all on the per-step kernels."""
+    rng = np.random.default_rng(3)
+    swarm = workloads.arena_balls(12, radius=3, arena=40, gap=0.5, sigma_v=0.3, steps=0, seed=7)
+    swarm.enable_cilia = 1
+    swarm.base_cilia, swarm.shift_cilia = rng.normal(0, 2e-4, (swarm.n_voxels, 3)), rng.normal(0, 2e-5, (swarm.n_voxels, 3))
+    swarm.enable_signals = 1
+    swarm.materials = [workloads.base_material(cte=0.0, cilia=1.0, matid=1),
+                       workloads.base_material(cte=0.0, cilia=1.0, matid=2, is_pacemaker=1, pacemaker_period=0.05)]
+    swarm.mat = (rng.random(swarm.n_voxels) < 0.05).astype(np.int32)
+    models = [workloads.drop(9, gap=1, shift=2, steps=0), swarm, workloads.slab(21, 10, 6, steps=0, collisions=True),
+              workloads.arena_balls(14, radius=3, arena=26, gap=0.0, sigma_v=0.4, steps=0, seed=5), workloads.cube(3, steps=0)]
+    got = []
+    for noalloc in (False, True):
+        b = engine.Batch(precision=precision, path=_abi.PATH_AUTO, collision_rebuild_interval=7, use_graph=graph, steps_per_launch=33)
+        s = [b.admit(m) for m in models]
+        for n in (6, 100, 3, 1, 70, 6, 64):
+            (b.step_noalloc if noalloc else b.step)(n)
+            st = b.poll()
+        assert all(st[x].steps == 250 for x in s)
+        got.append([b.read_state(x) for x in s])
+        b.close()
+    for x, y in zip(*got):
+        for k in ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac"):
+            assert np.array_equal(x[k], y[k]), k
