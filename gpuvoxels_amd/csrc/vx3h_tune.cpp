@@ -8,13 +8,14 @@
 // beyond the staleness rule add only watched pairs that cannot touch in between).
 // Every candidate runs the same simulations from their initial state in a fresh
 // batch: warm-up steps, then timed steps between two synchronizations; the fastest
-// in voxel-steps per second wins.
+// in voxel-steps per second wins (chooseTrial).
 #include <algorithm>
 #include <chrono>
 #include <vector>
 
 #include "../../include/vx3h.h"
 #include "vx3h_internal.h"
+#include "vx3h_tune.h"
 
 using vx3::g_err;
 
@@ -78,8 +79,7 @@ extern "C" vx3h_status vx3h_autotune(int device, const vx3h_sim_desc* const* des
     std::vector<int> intervals = {base->collision_rebuild_interval};
     if (tune_rebuild_interval && collisions) intervals = {0, 4, 8, 16};
 
-    int count = 0;
-    double bestRate = -1;
+    std::vector<vx3h_tune_trial> all;
     for (int bs : blocks)
         for (int spl : spls)
             for (int iv : intervals) {
@@ -90,10 +90,14 @@ extern "C" vx3h_status vx3h_autotune(int device, const vx3h_sim_desc* const* des
                 double rate = 0;
                 vx3h_status st = trial(device, descs, n_descs, c, warmup_steps, trial_steps, &rate);
                 if (st != VX3H_OK) return st;
-                if (trials && count < cap) trials[count] = vx3h_tune_trial{bs, spl, iv, rate};
-                count++;
-                if (rate > bestRate) { bestRate = rate; *best = c; }
+                all.push_back(vx3h_tune_trial{bs, spl, iv, rate});
+                if (trials && (int)all.size() <= cap) trials[all.size() - 1] = all.back();
             }
-    if (n_trials) *n_trials = count;
+    const vx3h_tune_trial& won = all[vx3::chooseTrial(all)];
+    *best = *base;
+    best->block_size = won.block_size;
+    best->steps_per_launch = won.steps_per_launch;
+    best->collision_rebuild_interval = won.collision_rebuild_interval;
+    if (n_trials) *n_trials = (int)all.size();
     return VX3H_OK;
 }

@@ -430,7 +430,8 @@ vx3h_status vx3h_sim_collision_pairs(vx3h_batch* b, int slot, int* pairs, int ca
  * (VX3_VoxelyzeKernel.cu:259-269,566-623).  Runs the given simulations from their
  * initial state once per candidate configuration, in a fresh batch on `device`:
  * warmup_steps untimed, then trial_steps timed; *best receives the fastest (in
- * voxel-steps/s) of base with block_size in {0, 128, 256, 512 (, 1024 for F32)},
+ * voxel-steps/s) of base with block_size in {0, 128, 256, 512 (, 1024 for F32)} (not 0 only
+ * if that is more than 2% faster: a given size leaves kernels that choose theirs out),
  * steps_per_launch in {250, 500, 1000, 2000} and, only when tune_rebuild_interval is
  * set and some simulation has collisions, collision_rebuild_interval in
  * {0, 4, 8, 16}.  None of them changes a result: the first two only decide which
