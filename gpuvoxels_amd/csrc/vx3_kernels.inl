@@ -12,6 +12,7 @@
 //   k_control   per simulation: step count, divergence, periodic FP64 center of
 //               mass, time advance, stop condition
 #include "vx3_batch.h"
+#include "vx3_pair.h"
 #include "vx3_physics.h"
 #include "vx3_powf.h"
 
@@ -679,16 +680,6 @@ __global__ void __launch_bounds__(256) k_col_list(DevBatch<real> b) {
 }
 
 
-// True only for pairs whose contact force is zero (pairContact's rel <= 0), without its square
-// root and divisions: most watched pairs most of the time.  The margin covers the rounding of
-// the contact distance and of the length (a few parts in 2^24); a distance whose square may have
-// lost bits to underflow decides nothing, nor does a NaN.
-__device__ __forceinline__ bool pairApart(real xi, real yi, real zi, real xj, real yj, real zj, float tfi, float tfj, real nom) {
-    const float ox = (float)(xj - xi), oy = (float)(yj - yi), oz = (float)(zj - zi);
-    const float reach = (float)nom * (tfi + tfj) * 0.625f, r2 = reach * reach;
-    return ox * ox + oy * oy + oz * oz > r2 * (1.0f + 0x1p-18f) && r2 > 1e-30f;
-}
-
 // Contact force of the pair (i, j), i the lower index, on voxel i: CVX_Collision::
 // updateContactForce (VX_Collision.cpp:41-56) from both voxels' pre-step position,
 // momentum and thermal factor.  Shared by the per-step and resident kernels.
@@ -698,8 +689,7 @@ __device__ __forceinline__ void pairContact(const VoxMatDev& m1, const VoxMatDev
     const float kp = 2.0f / (1.0f / m1.penetrationStiffness + 1.0f / m2.penetrationStiffness);
     const float cd = 0.5f * (m1.zetaCollision * m1.c2xSqMxExS + m2.zetaCollision * m2.c2xSqMxExS);
     const float ox = (float)(pjx - pix), oy = (float)(pjy - piy), oz = (float)(pjz - piz);
-    const real b1 = nom * (real)tfi, b2 = nom * (real)tfj;
-    const float nomDist = (float)(((b1 + b1 + b1) / (real)3.0f + (b2 + b2 + b2) / (real)3.0f) * (real)0.625f);
+    const float nomDist = pairDistance<real>(tfi, tfj, nom);
     const float len = sqrtf(ox * ox + oy * oy + oz * oz);
     const float rel = nomDist - len;
     fx = fy = fz = 0;
