@@ -319,3 +319,55 @@ def test_beside_the_per_step_kernels(precision, graph):
     for x, y in zip(*got):
         for k in ("pos", "orient", "lin_mom", "ang_mom", "flags", "tfac"):
             assert np.array_equal(x[k], y[k]), k
+
+
+def bodies(cells, watch):
+    """One simulation of the given lattice cells (connected ones are bodies)."""
+    m = workloads.drop(4, gap=1, shift=0, steps=0)
+    m.ijk = cells[np.lexsort((cells[:, 0], cells[:, 1], cells[:, 2]))].astype(np.int32)
+    m.mat, m.phase, m.watch_distance = np.zeros(len(cells), np.int32), None, watch
+    return m
+
+
+def lattice(n, pitch):
+    g = np.arange(n) * pitch
+    return np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+
+
+def partners(m, pairs):
+    return np.bincount(pairs.ravel(), minlength=m.n_voxels)
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+@pytest.mark.parametrize("side,watch", [(7, 2.5), (8, 3.5), (11, 3.0)])
+def test_lists_just_past_the_column(precision, side, watch):
+    """Two plates face to face, a tile each, whose voxels watch a few more partners than an LDS
+    column holds: those past it, up to 512 a tile, are merged in without a second walk."""
+    y, x = (a.ravel() for a in np.meshgrid(np.arange(side), np.arange(side), indexing="ij"))
+    plate = np.stack([x, y, 0 * x], 1)
+    m = bodies(np.concatenate([plate, plate + [0, 0, 2]]), watch)
+    a, c = (run([m], [8], k, precision) for k in (False, True))
+    past = np.maximum(partners(m, c[0][1]) - 36, 0)
+    for top in (0, 1):
+        assert 0 < past[(m.ijk[:, 2] > 0) == top].sum() <= 512
+    assert_equal(a, c)
+
+
+def test_more_candidates_than_one_walk_lists():
+    """Lone voxels within reach of a tile by the thousand."""
+    m = bodies(lattice(14, 2), 8.5)
+    a, c = (run([m], [8], k, _abi.PREC_F64) for k in (False, True))
+    # a tile holds 64 voxels: 4 x 4 x 4 of them reach as far as 10 voxels beyond on every side
+    assert m.n_voxels == 2744 and (3 * 2 + 1 + 20) ** 3 / 8 > 2048 and partners(m, c[0][1]).max() > 400
+    assert_equal(a, c)
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+def test_more_tiles_in_reach_than_one_gather_holds(precision):
+    """Lone voxels so far apart that each has a tile, with a watch radius that takes in more
+    than 512 of them: the tiles in reach are walked a few at a time."""
+    m = bodies(lattice(10, 20), 98.5)
+    a, c = (run([m], [8], k, precision) for k in (False, True))
+    box = (np.abs(m.ijk[:, None] - m.ijk[None]) <= 100).all(-1).sum(1)
+    assert box.max() > 512 and partners(m, c[0][1]).max() > 300
+    assert_equal(a, c)
