@@ -78,20 +78,30 @@ struct Planner {
                 lo[a] = std::min(lo[a], ijk[3 * part[i] + a]);
                 hi[a] = std::max(hi[a], ijk[3 * part[i] + a]);
             }
+        auto extent = [&](int a) { return (long long)hi[a] - lo[a] + 1; };
         int ax = 0;
-        for (int a = 1; a < 3; a++) if (hi[a] - lo[a] > hi[ax] - lo[ax]) ax = a;
+        for (int a = 1; a < 3; a++) if (extent(a) > extent(ax)) ax = a;
         const int kl = k / 2;
         size_t m = (size_t)((double)n * kl / k + 0.5);
         m = std::max<size_t>(1, std::min(m, n - 1));
         // the m lowest along the axis, ties in the order they come (by voxel index): a histogram of
-        // the coordinate finds the cut, so a level costs two passes and keeps the order
-        count.assign(hi[ax] - lo[ax] + 1, 0);
-        for (size_t i = 0; i < n; i++) count[ijk[3 * part[i] + ax] - lo[ax]]++;
+        // the coordinate finds the cut, so a level costs two passes and keeps the order.  (Where
+        // bodies lie far apart it would be longer than the voxels are many: a selection instead.)
         int at = 0;
         size_t below = 0;
-        while (below + count[at] < m) below += count[at++];
+        if (extent(ax) <= 4 * (long long)n + 1024) {
+            count.assign(extent(ax), 0);
+            for (size_t i = 0; i < n; i++) count[ijk[3 * part[i] + ax] - lo[ax]]++;
+            while (below + count[at] < m) below += count[at++];
+            at += lo[ax];
+        } else {
+            count.resize(n);
+            for (size_t i = 0; i < n; i++) count[i] = ijk[3 * part[i] + ax];
+            std::nth_element(count.begin(), count.begin() + (m - 1), count.end());
+            at = count[m - 1];
+            for (size_t i = 0; i < m - 1; i++) below += count[i] < at;
+        }
         size_t ties = m - below, j = 0, r = 0;
-        at += lo[ax];
         aside.resize(std::max(aside.size(), n));
         for (size_t i = 0; i < n; i++) {
             const int v = part[i], c = ijk[3 * v + ax];
