@@ -1331,6 +1331,18 @@ struct PreparedSim {
     StepTilePlan stepPlan;
 };
 
+// whether a model's physics, its number of phases aside, is what the resident and the fused
+// kernels compute; the rest runs on the per-step kernels
+bool plainPhysics(const vx3h_sim_desc* desc, const HostModel& H) {
+    // VoxCAD stop conditions and equilibrium mode are evaluated by the stream path's control pass
+    if (desc->stop_condition_type != VX3H_SC_NONE || desc->equilibrium_mode != 0) return false;
+    if (H.collisions)   // target contacts (hit counts) are counted by the per-step kernels
+        for (int i = 0; i < desc->n_materials; i++)
+            if (desc->materials[i].is_target) return false;
+    return (int)H.vmats.size() <= RES_MAX_VMATS && (int)H.lmats.size() <= RES_MAX_LMATS && !H.extras() && !desc->enable_detach &&
+           !desc->secondary_experiment && !desc->enable_signals && !desc->enable_attach && !(desc->max_dist_close_pairs > 0);
+}
+
 bool stepPlanOf(const vx3h_batch* b, const HostModel& H, StepTilePlan* out) {
     std::vector<char> interior(H.nv);
     for (int v = 0; v < H.nv; v++) interior[v] = (H.vflags[v] & VF_INTERIOR) != 0;
@@ -1362,7 +1374,8 @@ vx3h_status prepareSim(const vx3h_batch* b, const vx3h_sim_desc* desc, PreparedS
         }
     }
     // too large for the resident kernels: the step tiles, where admission may use them
-    if (H.nv > 0 && b->tiledShape >= 0 && !(p->planned && p->planOk && p->plan.tiles.size() > 1)) {
+    if (H.nv > 0 && b->tiledShape >= 0 && b->cfg.path != VX3H_PATH_RESIDENT && plainPhysics(desc, H) &&
+        !(p->planned && p->planOk && p->plan.tiles.size() > 1)) {
         const ResidentShapeInfo& r = b->shapes[b->tiledShape];
         int perAxis[3] = {0, 0, 0};
         for (int i = 0; i < H.nl; i++) perAxis[H.laxis[i]]++;
@@ -1584,9 +1597,7 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
     bool targets = false;   // target contacts (hit counts) are counted by the per-step kernels
     if (H.collisions)
         for (int i = 0; i < desc->n_materials; i++) targets |= desc->materials[i].is_target != 0;
-    const bool resOk = (int)H.vmats.size() <= RES_MAX_VMATS && (int)H.lmats.size() <= RES_MAX_LMATS &&
-                       nPhases <= RES_MAX_PHASES && !voxcad && !H.extras() && !desc->enable_detach &&
-                       !desc->secondary_experiment && !desc->enable_signals && !attach && !closePairs && !targets;
+    const bool resOk = NV > 0 && nPhases <= RES_MAX_PHASES && plainPhysics(desc, H);
     if (b->cfg.path != VX3H_PATH_STREAM && NV > 0 && resOk) {
         for (int si : b->shapePref) {
             const ResidentShapeInfo& r = b->shapes[si];
