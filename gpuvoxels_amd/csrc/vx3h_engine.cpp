@@ -84,10 +84,11 @@ struct SlotHost {
     int nlSeen = 0;              // links known to the host shadows below (nl + attached ones read back)
     int shape = -1;              // resident kernel shape, -1 = stream path (or tiled)
     int tiles = 0;               // > 0: runs on the tiled resident kernel as this many workgroups
-    TilePlan tplan, fplan;       // its tiles (sim-local): for the axis-by-axis kernel, and finer ones (planned when first
-                                 // used) for the kernel with the links of all axes at once
-    int fineSlots = 0;           // owned and halo voxels of a tile that fplan was planned for (0: not yet)
-    TilePlace tplace, fplace;    // their tables: the first from admission on, the finer ones beside them once used
+    TilePlan tplan;              // its tiles (sim-local): for the axis-by-axis kernel,
+    TilePlan fplan[2];           // and finer ones for the kernel with the links of all axes at once, of two sizes
+    bool fplanned[2] = {};       // (planned when first used; see chooseTiles), of which
+    int fuse = 0;                // it uses these
+    TilePlace tplace, fplace[2]; // their tables: the first from admission on, the finer ones beside them once used
     bool oneTile = false;        // a one-workgroup simulation with one-tile tables in the pools
     int axisLinks = 0;           // links on its busiest axis
     std::vector<TsTile> stepTiles;   // steps on the fused per-step kernel as these tiles
@@ -706,7 +707,9 @@ vx3h_status ensureOneTile(vx3h_batch* b, int s) {
 // smaller (the loads of all their links share LDS), so that is done while one launch holds all
 // of them and nothing else shares the chip; else fewer, larger tiles get more done.  Plans of
 // 448 slots a tile where these fit too (2.6 times the tiles), else as large as the shape takes
-// (1.6 to 2.1 times): still smaller ones wait for as many more barriers as they save.  Measured
+// (1.6 to 2.1 times): still smaller ones wait for as many more barriers as they save.  A plan
+// takes milliseconds, so a simulation keeps those it has had, and one that was planned among
+// others keeps its larger ones when they leave.  Measured
 // on MI355X, us per step, the shape's own size -> 448 slots; axis by axis in brackets:
 //                                        FP32                     FP64
 //   one robot on a 14^3 grid       9.2 -> 9.0 (13.8)       12.0 -> 10.8 (19.8)
@@ -720,36 +723,48 @@ vx3h_status chooseTiles(vx3h_batch* b) {
     size_t coarse = 0, tiles = 0;
     for (int s : b->tiledSims) coarse += b->slots[s].tplan.tiles.size();
     fine = fine && 3 * coarse <= 2 * cap;
-    const int slots = std::min(5 * coarse <= 2 * cap ? 448 : INT32_MAX, b->fineShape.block);
-    for (size_t i = 0; fine && i < b->tiledSims.size(); i++) {
-        SlotHost& sh = b->slots[b->tiledSims[i]];
-        if (sh.fineSlots != slots) {
+    const int want = 5 * coarse <= 2 * cap ? 0 : 1;
+    auto planned = [&](SlotHost& sh, int k) -> size_t {   // tiles of plan k, made when first asked for; 0: none fits
+        if (!sh.fplanned[k]) {
             std::vector<int> axis(sh.nl);
             for (int v = 0; v < sh.nv; v++)
                 for (int a = 0; a < 3; a++) {
                     const int l = sh.vlinks[6 * (size_t)v + 2 * a];
                     if (l >= 0) axis[l] = a;
                 }
-            TilePlan p;
-            if (!planTiles(sh.nv, sh.ijk.data(), sh.nl, sh.lneg.data(), sh.lpos.data(), axis.data(), slots, b->fineShape.links / 3,
-                           b->fineCap, &p, false))
-                p = TilePlan();
-            HIPCHK(hipStreamSynchronize(b->stream));   // launches that read the old plan's tables
-            releaseTiles(b, sh.fplace);
-            sh.fplan = std::move(p);
-            sh.fineSlots = slots;
+            if (!planTiles(sh.nv, sh.ijk.data(), sh.nl, sh.lneg.data(), sh.lpos.data(), axis.data(),
+                           std::min(k ? INT32_MAX : 448, b->fineShape.block), b->fineShape.links / 3, b->fineCap, &sh.fplan[k], false))
+                sh.fplan[k] = TilePlan();
+            sh.fplanned[k] = true;
         }
-        tiles += sh.fplan.tiles.size();
-        fine = sh.fplan.tiles.size() > 1 && tiles <= cap;
-    }
+        return sh.fplan[k].tiles.size() > 1 ? sh.fplan[k].tiles.size() : 0;
+    };
     for (size_t i = 0; fine && i < b->tiledSims.size(); i++) {
         SlotHost& sh = b->slots[b->tiledSims[i]];
-        if (sh.fplace.tiles || placeTiles(b, sh.fplan, &sh.fplace) == VX3H_OK) continue;
+        sh.fuse = want == 0 && !sh.fplanned[0] && sh.fplanned[1] ? 1 : want;
+        const size_t n = planned(sh, sh.fuse);
+        tiles += n;
+        fine = n > 0;
+    }
+    for (size_t i = 0; fine && tiles > cap && i < b->tiledSims.size(); i++) {   // too many: the larger ones
+        SlotHost& sh = b->slots[b->tiledSims[i]];
+        const size_t n = sh.fuse == 0 ? planned(sh, 1) : 0;
+        if (!n) continue;
+        tiles = tiles - sh.fplan[0].tiles.size() + n;
+        sh.fuse = 1;
+    }
+    fine = fine && tiles <= cap;
+    for (size_t i = 0; fine && i < b->tiledSims.size(); i++) {
+        SlotHost& sh = b->slots[b->tiledSims[i]];
+        if (sh.fplace[sh.fuse].tiles || placeTiles(b, sh.fplan[sh.fuse], &sh.fplace[sh.fuse]) == VX3H_OK) continue;
         fine = false;   // no device memory for them: the larger tiles stay
         (void)hipGetLastError();
     }
     b->fine = fine;
-    for (int s : b->tiledSims) b->slots[s].tiles = (int)(fine ? b->slots[s].fplan : b->slots[s].tplan).tiles.size();
+    for (int s : b->tiledSims) {
+        SlotHost& sh = b->slots[s];
+        sh.tiles = (int)(fine ? sh.fplan[sh.fuse] : sh.tplan).tiles.size();
+    }
     return VX3H_OK;
 }
 
@@ -797,8 +812,8 @@ vx3h_status syncTiles(vx3h_batch* b) {
         for (int s : bin) {
             const SlotHost& sh = b->slots[s];
             const bool fine = b->fine && sh.tiles;
-            const TilePlan& plan = fine ? sh.fplan : sh.tplan;
-            const TilePlace& at = fine ? sh.fplace : sh.tplace;
+            const TilePlan& plan = fine ? sh.fplan[sh.fuse] : sh.tplan;
+            const TilePlace& at = fine ? sh.fplace[sh.fuse] : sh.tplace;
             for (TileDesc d : plan.tiles) {
                 d.sim = s;
                 d.vOff += at.v0;
@@ -2596,7 +2611,7 @@ extern "C" vx3h_status vx3h_sim_retire(vx3h_batch* b, int slot) {
     }
     if (sh.tiles) {
         b->tiledSims.erase(std::remove(b->tiledSims.begin(), b->tiledSims.end(), slot), b->tiledSims.end());
-        releaseTiles(b, sh.fplace);
+        for (TilePlace& t : sh.fplace) releaseTiles(b, t);
         b->tileDirty = true;
     } else if (sh.shape >= 0) {
         auto& L = b->resLists[sh.shape];

@@ -79,3 +79,28 @@ def test_others_join_and_leave(precision):
     same(state(b, [s], [big]), state(c, [r], [big]))
     b.close()
     c.close()
+
+
+def test_plans_are_kept_as_others_leave():
+    """Simulations planned among others go on as the tiles they have when some leave (a plan takes
+    longer than it would save), and one that has had plans of both sizes goes back to the smaller."""
+    models = [robot(20 + i, 40) for i in range(3)]
+    b = engine.Batch(precision=_abi.PREC_F32, path=_abi.PATH_AUTO)
+    s = [b.admit(models[0])]
+    b.step(10)
+    alone = b.workgroups(s[0])
+    s += [b.admit(m) for m in models[1:]]
+    b.step(10)
+    among = [b.workgroups(x) for x in s]
+    assert 1 < among[0] < alone
+    b.retire(s[2])
+    b.step(10)
+    assert [b.workgroups(x) for x in s[:2]] == [alone, among[1]]
+    got = state(b, s[:2], models[:2])
+    b.close()
+    for i, n in ((0, 30), (1, 20)):
+        c = engine.Batch(precision=_abi.PREC_F32, path=_abi.PATH_STREAM)
+        r = c.admit(models[i])
+        c.step_noalloc(n)
+        same([got[i]], state(c, [r], [models[i]]))
+        c.close()
