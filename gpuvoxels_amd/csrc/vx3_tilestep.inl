@@ -20,10 +20,14 @@
 //
 // A step that cannot be taken (a collision table too small: TsReport::grow) or not as a whole
 // (a diverged link: its voxels do not move) is only known once every tile has run: the
-// control step then leaves the old copy current (SC_TSPARV, SC_TSPARL), so nothing has
-// happened but for the partner lists, or only the link pass has.  A running simulation's current copies are always
+// control step then leaves the old copy current (SC_TSPARV, SC_TSPARL, SC_TSTOP), so nothing
+// has happened, or only the link pass has.  A running simulation's current copies are always
 // those of the launch's parity, so a tile reads its state without waiting for the control
 // words.
+//
+// Two sets of partner lists take turns, one from the table's start on and one at its end; where
+// both do not fit, the entries of the older set are lost (which shows only where the new one is
+// not taken: see listsLost for a table that is too small).
 //
 // Collision lists (the pair rule of vx3_kernels.inl's k_col_list, the same lists): each tile
 // keeps the bounding boxes of its surface voxels, of all and of each wave's 64, as of the last
@@ -149,7 +153,10 @@ __device__ __forceinline__ void tsAdvance(const DevBatch<real>& b, const TsArgs&
         return;
     }
     c.steps++;
-    if ((f & SC_COLLISIONS) && (f & SC_REBUILD)) c.rebuilds++;
+    if ((f & SC_COLLISIONS) && (f & SC_REBUILD) && r.diverged != seq) {   // (its lists come after the links)
+        c.rebuilds++;
+        f ^= SC_TSTOP;
+    }
     f &= ~SC_REBUILD;
     if ((f & SC_COLLISIONS) && (r.stale == seq || (sc.colInterval > 0 && c.steps % sc.colInterval == 0))) f |= SC_REBUILD;
     f ^= SC_TSPARL;
@@ -209,7 +216,7 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) k_ts_load(DevBatch<real> b, TsAr
     __shared__ unsigned sMoved;
     if (tid == 0) sMoved = 0;
     __syncthreads();
-    char *const A = tsStat(ts, td.rec), *const C = tsState(ts, td.rec, 0);
+    char *const A = tsStat(ts, td.rec), *const C = tsState(ts, td.rec, 0), *const Q = A + (flags & SC_TSTOP ? TsA::LISTS : 0);
     float x = 0, y = 0, z = 0;
     const bool surf = tid < td.nSurf, col = (flags & SC_COLLISIONS) != 0;
     for (int i = tid; i < td.nOwn; i += VX3_TS_BLOCK) {
@@ -225,9 +232,9 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) k_ts_load(DevBatch<real> b, TsAr
         x = (float)b.px[g]; y = (float)b.py[g]; z = (float)b.pz[g];
         const float w[3] = {b.lastWatch[3 * g], b.lastWatch[3 * g + 1], b.lastWatch[3 * g + 2]};
 #pragma unroll
-        for (int k = 0; k < 3; k++) row<float>(A, TsA::LW + k * TsA::R4, i) = w[k];
-        row<int>(A, TsA::NBC, i) = b.nbCount[g];
-        row<int>(A, TsA::NBS, i) = b.nbStart[g];
+        for (int k = 0; k < 3; k++) row<float>(Q, TsA::LW + k * TsA::R4, i) = w[k];
+        row<int>(Q, TsA::NBC, i) = b.nbCount[g];
+        row<int>(Q, TsA::NBS, i) = b.nbStart[g];
         if (flags & SC_REBUILD) continue;
         const real dx = b.px[g] - (real)w[0], dy = b.py[g] - (real)w[1], dz = b.pz[g] - (real)w[2];
         const real d2 = dx * dx + dy * dy + dz * dz;
@@ -268,7 +275,7 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) k_ts_store(DevBatch<real> b, TsA
     tsAdvance(b, ts, td, sc, c, ts.report[(1 - ts.par) * ts.ctlCap + td.ctl], sQ, &sStop);
     const int tid = threadIdx.x;
     char *const A = tsStat(ts, td.rec), *const V = tsState(ts, td.rec, (c.flags & SC_TSPARV) != 0),
-         *const L = tsState(ts, td.rec, (c.flags & SC_TSPARL) != 0);
+         *const L = tsState(ts, td.rec, (c.flags & SC_TSPARL) != 0), *const Q = A + (c.flags & SC_TSTOP ? TsA::LISTS : 0);
     const bool col = (c.flags & SC_COLLISIONS) != 0;
     for (int i = tid; i < td.nOwn; i += VX3_TS_BLOCK) {
         const int g = row<int>(A, TsA::ORIG, i);
@@ -281,9 +288,9 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) k_ts_store(DevBatch<real> b, TsA
         b.vflags[g] = row<int>(V, TsS::VI, i);
         if (!col || i >= td.nSurf) continue;
 #pragma unroll
-        for (int k = 0; k < 3; k++) b.lastWatch[3 * g + k] = row<float>(A, TsA::LW + k * TsA::R4, i);
-        b.nbCount[g] = row<int>(A, TsA::NBC, i);
-        b.nbStart[g] = row<int>(A, TsA::NBS, i);
+        for (int k = 0; k < 3; k++) b.lastWatch[3 * g + k] = row<float>(Q, TsA::LW + k * TsA::R4, i);
+        b.nbCount[g] = row<int>(Q, TsA::NBC, i);
+        b.nbStart[g] = row<int>(Q, TsA::NBS, i);
     }
     for (int i = tid; i < td.nOwn; i += VX3_TS_BLOCK) {
 #pragma unroll
@@ -367,7 +374,8 @@ struct TsContacts {
 
 // The partner lists of the tile's surface voxels, from the old copy of the state; the whole
 // workgroup.  g: the thread's voxel (batch index), mine: it is on the surface.  Returns false
-// when the simulation's table is too small (no list is written then).  Writes the tile's boxes
+// when the simulation's table is too small (no list is written then).  top: these lists go to the
+// table's end and the second rows.  Writes the tile's boxes
 // into the new copy.
 //
 // Bound by instruction issue and LDS latency with one wave per SIMD (the last tile's rebuild
@@ -376,7 +384,7 @@ struct TsContacts {
 // of 123 voxels in FP32: 125,000 with every staged candidate tested by every voxel in turn,
 // distance and nearby set together; 57,000 with a wave's own reach and the two parts of match.
 // Staged candidates sorted into cells and walked voxel by voxel: slower than the first.
-__device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& ts, const TsT& td, SimCtl& sc, int* nbUsed,
+__device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& ts, const TsT& td, SimCtl& sc, int* nbUsed, bool top,
                                         bool mine, int g, unsigned char* smem, float (*sReach)[6]) {
     unsigned* sMask = (unsigned*)smem;                                     // [word][thread]
     short* sBit = (short*)(sMask + VX3_NEAR_WORDS * VX3_TS_BLOCK);
@@ -664,7 +672,7 @@ __device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& t
                 atomicMax(&sc.nbNeed, at + total);
                 at = -1;
             }
-            sBase = at;
+            sBase = at < 0 || !top ? at : sc.nbCap - at - total;
         }
         __syncthreads();
         if (sBase < 0) return false;
@@ -712,11 +720,12 @@ __device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& t
         break;
     }
     if (mine) {
-        row<int>(A, TsA::NBC, tid) = n;
-        row<int>(A, TsA::NBS, tid) = from;
-        row<float>(A, TsA::LW, tid) = (float)x;
-        row<float>(A, TsA::LW + TsA::R4, tid) = (float)y;
-        row<float>(A, TsA::LW + 2 * TsA::R4, tid) = (float)z;
+        char* const Q = A + (top ? TsA::LISTS : 0);
+        row<int>(Q, TsA::NBC, tid) = n;
+        row<int>(Q, TsA::NBS, tid) = from;
+        row<float>(Q, TsA::LW, tid) = (float)x;
+        row<float>(Q, TsA::LW + TsA::R4, tid) = (float)y;
+        row<float>(Q, TsA::LW + 2 * TsA::R4, tid) = (float)z;
         if (again)
             for (int i = 1; i < n; i++) {
                 const int c = out[i];
@@ -838,8 +847,10 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) __attribute__((amdgpu_waves_per_
     const float size = (float)uni(sc.voxSize);
     const float dtf = uni(sc.dt);
     if (tid == 0) sMoved = 0;
+    // the lists that this step uses: those at the table's end, or at its start
+    const bool top = ((flags & SC_TSTOP) != 0) != (col && (flags & SC_REBUILD));
     if (col && (flags & SC_REBUILD)) {
-        if (!tsLists(b, ts, td, sc, &report->nbUsed, surf, surf ? row<int>(A, TsA::ORIG, tid) : -1, smem, sBoxRed)) {
+        if (!tsLists(b, ts, td, sc, &report->nbUsed, top, surf, surf ? row<int>(A, TsA::ORIG, tid) : -1, smem, sBoxRed)) {
             if (tid == 0) tsSay(&report->grow, seq);
             return;   // no tile's step counts
         }
@@ -1060,9 +1071,10 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) __attribute__((amdgpu_waves_per_
                       row<real>(C, TsS::VR + 12 * TsS::RR, i));
         nc = 0;
         if (col && i < td.nSurf) {
-            nc = row<int>(A, TsA::NBC, i);
+            char* const Q = A + (top ? TsA::LISTS : 0);
+            nc = row<int>(Q, TsA::NBC, i);
 #pragma unroll
-            for (int k = 0; k < 3; k++) lw[k] = row<float>(A, TsA::LW + k * TsA::R4, i);
+            for (int k = 0; k < 3; k++) lw[k] = row<float>(Q, TsA::LW + k * TsA::R4, i);
         }
     };
     if (own) readRest(tid);
@@ -1097,7 +1109,7 @@ __global__ void __launch_bounds__(VX3_TS_BLOCK) __attribute__((amdgpu_waves_per_
                 con.o2p = ts.o2p + td.o0;
                 con.v = row<int>(A, TsA::ORIG, i);
                 con.v0 = sc.v0;
-                con.start = row<int>(A, TsA::NBS, i);
+                con.start = row<int>(A + (top ? TsA::LISTS : 0), TsA::NBS, i);
             }
             voxelStep<real>(m, ext, dtf, nom, ix, iy, iz, tf, fs, ms, con, pos, lm, o, am, vf);
         }

@@ -58,7 +58,8 @@ enum { SC_VARY = 1, SC_EXPANSION = 2, SC_DIVERGED_PENDING = 4, SC_POISSON = 8, S
        SC_TILESTEP = 1 << 22,      // steps on the fused per-step kernel (k_ts_step) in calls of several steps
        SC_TSLOADED = 1 << 23,      // TsCtl only: its state is in the fused kernel's tile arrays,
        SC_TSPARV = 1 << 24,        // which of the two copies of its voxel state is current,
-       SC_TSPARL = 1 << 25 };      // and of its link state
+       SC_TSPARL = 1 << 25,        // and of its link state
+       SC_TSTOP = 1 << 26 };       // its partner lists are those the fused kernel put at the table's end
 #define VX3_COL_HBLOCK 1024     // hash buckets per scan block; a simulation's buckets are whole blocks
 
 // A voxel's nearby set (the surface voxels within the link-hop radius) as a bit mask over
@@ -214,9 +215,7 @@ struct TsTile {
 #define VX3_TS_SLOT_BITS 9
 
 // A tile record: rows of VX3_TS_OWN elements, one per owned slot.  TsStat (byte offsets) is
-// written at admission up to ST_END; the rest and TsState belong to a call.  What a step that is
-// not taken (TsReport::grow) may have overwritten in TsStat, the lists and what goes with them,
-// is rebuilt by the step that is taken in its place.
+// written at admission up to ST_END; the rest and TsState belong to a call.
 struct TsStat {
     static constexpr int R4 = 4 * VX3_TS_OWN;
     static constexpr int ST = 0;               // voxel material | phase << 4 | external << 10 | link material of axis a << (12 + 4a)
@@ -230,7 +229,8 @@ struct TsStat {
     static constexpr int ST_END = IJK + 2 * R4;
     static constexpr int LW = ST_END;          // 3 rows: position at the last list rebuild
     static constexpr int NBC = LW + 3 * R4, NBS = NBC + R4;   // partner list: entries, start in nbList
-    static constexpr int BYTES = (NBS + R4 + 255) / 256 * 256;
+    static constexpr int LISTS = 5 * R4;       // these rows, and once more (SC_TSTOP: the second are current)
+    static constexpr int BYTES = (LW + 2 * LISTS + 255) / 256 * 256;
 };
 template <int REAL> struct TsState {   // one of the two copies; REAL = bytes of the state precision
     static constexpr int RR = REAL * VX3_TS_OWN, R4 = 4 * VX3_TS_OWN;

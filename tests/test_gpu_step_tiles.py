@@ -371,3 +371,20 @@ def test_more_tiles_in_reach_than_one_gather_holds(precision):
     box = (np.abs(m.ijk[:, None] - m.ijk[None]) <= 100).all(-1).sum(1)
     assert box.max() > 512 and partners(m, c[0][1]).max() > 300
     assert_equal(a, c)
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+def test_divergence_in_a_step_that_rebuilds_lists(precision):
+    """Lists rebuilt every step: a step that diverges ends before its lists come into use, so the
+    pairs of the simulation are those of the step before."""
+    m = workloads.arena_balls(20, radius=2, arena=22, gap=0.0, sigma_v=8.0, steps=0, seed=5)
+    one = np.flatnonzero(np.all(m.init_velocity == m.init_velocity[0], axis=1))
+    m.init_velocity[one] = np.random.default_rng(8).normal(0, 300.0, (len(one), 3))
+    a, c = (run([m], [400], k, precision, 1) for k in (False, True))
+    assert a[0][2].state == _abi.SIM_DIVERGED and len(c[0][1]) > 0
+    assert_equal(a, c)
+    b = engine.Batch(precision=precision, path=_abi.PATH_STREAM, collision_rebuild_interval=1)
+    s = b.admit(m)
+    b.step_noalloc(a[0][2].steps - 2)
+    assert not np.array_equal(b.collision_pairs(s), c[0][1])   # (they change from step to step)
+    b.close()
