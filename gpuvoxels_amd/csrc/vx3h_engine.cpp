@@ -1973,8 +1973,7 @@ extern "C" vx3h_status vx3h_batch_step(vx3h_batch* b, int n_steps) {
     // The fused kernel takes its simulations in calls of enough steps to pay for copying the
     // state into the tile arrays and back; shorter calls leave them to the per-step kernels,
     // and so does the first step of a simulation that stood still after its link pass.
-    const bool resume = b->resumePending;
-    b->resumePending = false;   // every waiting simulation resumes in the first step below
+    const bool resume = b->resumePending;   // every waiting simulation resumes in the first step below
     const bool fused = n_steps >= VX3_TS_MIN_STEPS && fusedSteps(b);
     if (fused)
         if (vx3h_status st = syncStep(b)) return st;
@@ -2020,6 +2019,7 @@ extern "C" vx3h_status vx3h_batch_step(vx3h_batch* b, int n_steps) {
         // the main stream waits for the resident launches, also after a failure
         const vx3h_status js = joinResident(b);
         if (!st) st = js;
+        if (!st) b->resumePending = false;
         done += c;
     }
     if (loaded) {
