@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from gpuvoxels_amd import _abi, engine, workloads
+from gpuvoxels_amd.model import MT
 
 pytestmark = pytest.mark.gpu
 
@@ -104,3 +105,30 @@ def test_plans_are_kept_as_others_leave():
         c.step_noalloc(n)
         same([got[i]], state(c, [r], [models[i]]))
         c.close()
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_F64, _abi.PREC_F32])
+def test_divergence_and_stop(precision):
+    """Simulations flung apart (large-angle links, then a diverged one: the launch is run again up
+    to that step), stopped by their step budget within a launch, and by a condition."""
+    def models():
+        ms = [robot(30 + i, 17) for i in range(3)]
+        rng = np.random.default_rng(8)
+        ms[0].init_velocity = rng.normal(0, 300.0, (ms[0].n_voxels, 3))
+        ms[1].init_velocity = rng.normal(0, 3.0, (ms[1].n_voxels, 3))
+        ms[1].max_steps = 77
+        ms[2].stop_tokens = [(MT["mtCONST"], 0.001), (MT["mtVAR"], 4.0), (MT["mtGREATERTHAN"], 0.0), (MT["mtEND"], 0.0)]
+        return ms
+    got = []
+    for noalloc in (False, True):
+        ms = models()
+        b = engine.Batch(precision=precision, path=_abi.PATH_AUTO, steps_per_launch=60)
+        s = [b.admit(m) for m in ms]
+        (b.step_noalloc if noalloc else b.step)(150)
+        if not noalloc:
+            assert all(b.workgroups(x) > 1 for x in s)
+        got.append(state(b, s, ms))
+        b.close()
+    assert [x[1].state for x in got[0]] == [_abi.SIM_DIVERGED, _abi.SIM_DONE, _abi.SIM_DONE]
+    assert np.any(got[0][1][0]["small_angle"] == 0)
+    same(*got)
