@@ -274,6 +274,8 @@ def config_leg(model, precision, steps, interval=0, kernel_steps=50, warmup=10):
     wg = [b.workgroups(x) for x in slots]
     kt = b.kernel_times(kernel_steps) if kernel_steps else {}
     b.close()
+    if "resident" in kt and not sum(wg):   # no resident kernel ran: the fused per-step kernel's time, per step
+        kt["fused"] = kt.pop("resident") / kernel_steps
     out = {"value": V * steps / dt, "unit": "voxel-steps/s", "voxels": V, "links": L, "steps": steps,
            "sims": len(models), "ms_per_step": dt / steps * 1e3, "dtype": "f64" if f64 else "f32", "admit_s": admit_s,
            "state": int(st.state), "steps_done": int(min(sts[x].steps for x in slots)), "kernel_ms": kt,

@@ -42,7 +42,8 @@ template <int BS, int LPT, int LMAX, bool TILED = false> struct ResidentAllShape
 //   one cube of 7^3, 9^3       11.1 -> 8.0     11.4 -> 9.7     (two rounds)
 //   200 robots on 8^3 grids    12.3 -> 6.1     10.4 -> 5.4
 //   200 robots on 10^3 grids   13.5 -> 9.1     10.9 -> 6.8
-//   512 robots on 12^3 grids         -         22.4 -> 17.1
+//   512 robots on 12^3 grids         -         22.3 -> 17.3   (first 3,000 steps; over 8,000, with
+//                                              24.7 -> 18.7    ever more links at large angles)
 template <int BS, int LPT, int LMAX, bool TILED = false>
 __global__ void __launch_bounds__(BS) k_resident_all(DevBatch<real> b, const int* simList, int nSteps, TileArgs ta) {
     typedef ResidentAllShape<BS, LPT, LMAX, TILED> Shape;

@@ -748,7 +748,7 @@ __device__ __forceinline__ bool tsLists(const DevBatch<real>& b, const TsArgs& t
 // loads issued before the control words they do not depend on.  Measured on MI355X, us per step
 // in one call of many, per-step kernels -> this kernel:
 //   64x64x32 cuboid, FP64, collisions (131,072 voxels)     66 -> 42
-//   64x64x1 plate, FP32, collisions                        30 -> 22
+//   61x47x7 plate, FP32, collisions                        30 -> 22
 //   2,048 balls of 257 voxels, FP64, rebuilt every 8      337 -> 141
 //   300 balls of 123 voxels, FP32, rebuilt every 8         62 -> 23
 template <int S, int N>

@@ -587,7 +587,7 @@ vx3h_status ensureGraph(vx3h_batch* b, int steps, int solo) {
 // units, each in its smallest shape, or when the axis-by-axis shapes they would take hold a
 // unit each too, all in one shape (workgroups go round the chip's eight dies kernel by kernel,
 // so two kernels' remainders can leave one die a round more: 512 robots in FP32, 23.5 us a step
-// in two shapes, 17.1 in one, 22.4 axis by axis).  Past that line more workgroups a unit win:
+// in two shapes, 17.1 in one, 22.4 axis by axis, in their first steps).  Past that line more workgroups a unit win:
 // 300 robots on 10^3 grids, FP32, 11.5 us a step axis by axis, 17.2 here; 512, 13.6 and 18.7.
 vx3h_status syncResLists(vx3h_batch* b) {
     if (!b->resDirty) return VX3H_OK;
@@ -1952,7 +1952,8 @@ vx3h_status admitPrepared(vx3h_batch* b, const vx3h_sim_desc* desc, PreparedSim*
 // MI355X, us per call, per-step kernels -> fused:
 //   steps                               4             5             6             8
 //   64x64x32, FP64, collisions    272 -> 253    337 -> 290    406 -> 327    532 -> 400
-//   64x64x1, FP32                 131 -> 137    160 -> 160    189 -> 180    248 -> 225
+//   61x47x7, FP32, collisions     135 -> 142    164 -> 166    192 -> 186    252 -> 229
+//   64x64x1, FP32, collisions     114 -> 112    139 -> 130    163 -> 148    213 -> 186
 //   2,048 balls of 257, FP64      962 -> 996            - (a list rebuild)
 //   300 balls of 123, FP32        141 -> 135            -     446 -> 199    513 -> 240
 #define VX3_TS_MIN_STEPS 6

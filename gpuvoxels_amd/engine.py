@@ -280,7 +280,8 @@ class Batch:
 
     def kernel_times(self, n_steps):
         """Mean per-pass kernel durations (ms) over n_steps steps, from HIP events
-        recorded on the batch's stream."""
+        recorded on the batch's stream; "resident": all n_steps steps of the resident,
+        tiled and fused kernels."""
         out = (C.c_double * len(self.PASSES))()
         check(lib().vx3h_batch_kernel_times(self.h, int(n_steps), out))
         return {k: out[i] for i, k in enumerate(self.PASSES) if out[i] > 0}

@@ -394,13 +394,14 @@ vx3h_status vx3h_build_topology(const vx3h_sim_desc* desc, vx3h_topology_view* v
  * steps without graph capture, with HIP events recorded on the batch's stream
  * around every kernel pass, and returns each pass's mean duration in ms
  * (avg_ms[k], k = 0 Poisson (now part of the voxel pass: always 0), 1 links,
- * 2 contacts, 3 voxels, 4 control, 5 resident multi-step kernel; 0 when the pass
- * did not run). */
+ * 2 contacts, 3 voxels, 4 control; 0 when the pass did not run) and, in avg_ms[5],
+ * the summed duration of the n_steps steps on the kernels without those passes: the
+ * resident and tiled ones' launches and the fused per-step kernel's. */
 #define VX3H_N_PASSES 6
 vx3h_status vx3h_batch_kernel_times(vx3h_batch* b, int n_steps, double* avg_ms);
 
 /* Which kernels step a simulation (no counterpart in the reference, which has one
- * path): *workgroups = 0 for the per-step kernels, 1 for one workgroup of the resident
+ * path): *workgroups = 0 for the per-step kernels (the fused one among them), 1 for one workgroup of the resident
  * kernel, n > 1 for n tiles of the tiled resident kernel (as of the last stepping call: a
  * simulation that has the device to itself runs as more, smaller tiles). */
 vx3h_status vx3h_sim_workgroups(vx3h_batch* b, int slot, int* workgroups);
